@@ -345,6 +345,12 @@ int Sim::flush_diag(std::vector<DiagGate> &window)
 {
     if (window.empty())
         return OK;
+    if (use_small_)
+    {
+        const int src = small_.window(ctx_, dstate_, window.data(), window.size());
+        window.clear();
+        return src;
+    }
     ZXA_TRY(flush_group());
     if (!wide_u3_.empty())
         return flush_wide(&window);
@@ -525,6 +531,12 @@ bool Sim::take_fan(unsigned t, GateFan &fan)
 // the first (applied after it).
 int Sim::emit_u3(std::vector<U3Gate> &descs)
 {
+    if (use_small_)
+    {
+        for (const U3Gate &g : descs)
+            ZXA_TRY(small_.gate(ctx_, dstate_, g));
+        return OK;
+    }
     bool simple = fusable();
     for (const U3Gate &g : descs)
     {
@@ -732,6 +744,12 @@ int Sim::execute()
     pass_has_fan_ = false;
     exp_group_.clear();
     wide_u3_.clear();
+    use_small_ = policy_ == POLICY_FUSED && M_ <= small_max_bits(prec_);
+    if (use_small_)
+    {
+        fresh_ = false; // the circuit's first run forms |0...0>
+        small_.begin(unsigned(M_), prec_);
+    }
 
     // Scheduling.  The reference policy batches each run of consecutive U3
     // gates and flushes the diagonal window when a run starts (zxh.cpp:440-470).
@@ -892,6 +910,11 @@ int Sim::execute()
                     eg.u[2 * i] = u[i].real();
                     eg.u[2 * i + 1] = u[i].imag();
                 }
+                if (use_small_)
+                {
+                    ZXA_TRY(small_.gate(ctx_, dstate_, eg));
+                    continue;
+                }
                 // the new bit is the top one and its half still zero
                 const bool top = eg.delta == uint64_t(1) << (active_bits() - 1);
                 if (stream && top && !exp_group_.empty() &&
@@ -954,6 +977,11 @@ int Sim::execute()
                 const uint64_t d = solve_expand(g.q, &rc);
                 if (rc)
                     return rc;
+                if (use_small_)
+                {
+                    ZXA_TRY(small_.swap(ctx_, dstate_, d & low_mask(active_bits()), local_selector(g.q), nullptr));
+                    break;
+                }
                 ZXA_TRY(flush_group());
                 ZXA_TRY(settle());
                 ZXA_TRY(x_apply(ctx_, dstate_, prec_, active_bits(), d & low_mask(active_bits()),
@@ -971,6 +999,12 @@ int Sim::execute()
                 const uint64_t d = solve_expand(g.q, &rc);
                 if (rc)
                     return rc;
+                if (use_small_)
+                {
+                    const uint64_t scq = local_selector(g.cq);
+                    ZXA_TRY(small_.swap(ctx_, dstate_, d & low_mask(active_bits()), local_selector(g.q), &scq));
+                    break;
+                }
                 ZXA_TRY(flush_group());
                 ZXA_TRY(settle());
                 ZXA_TRY(cx_apply(ctx_, dstate_, prec_, active_bits(), d & low_mask(active_bits()),
@@ -1007,6 +1041,8 @@ int Sim::execute()
         }
     }
     ZXA_TRY(flush_all());
+    if (use_small_)
+        ZXA_TRY(small_.run(ctx_, dstate_));
     ZXA_TRY(flush_pass());
     ZXA_TRY(flush_group());
     ZXA_TRY(settle());

@@ -10,6 +10,7 @@
 #pragma once
 
 #include "dev.h"
+#include "small.h"
 
 #include <complex>
 #include <cstdint>
@@ -186,6 +187,10 @@ class Sim
     std::vector<U3Gate> exp_group_;
     unsigned exp_base_ = 0;
     int flush_group();
+    // fused policy, a state that fits one compute unit's LDS: every
+    // operation goes to small_ and runs at the end of execute()
+    bool use_small_ = false;
+    SmallCircuit small_;
     Ctx ctx_;
 };
 
