@@ -419,6 +419,11 @@ int zero_fill(Ctx &ctx, void *p, size_t bytes);
 int set_ones(Ctx &ctx, const uint64_t *dstates, int count, int prec);
 // out (host) = the amplitudes at idx[0..count) of a 2^n state (synchronous).
 int gather(Ctx &ctx, const void *state, int prec, unsigned n, const uint64_t *idx, size_t count, void *out);
+// out (host, 2^(n + 1) doubles) = the virtual state in bit-reversed order
+// times f: amplitude A x ^ b of n qubits is f psi[x] (rows[q] bit c =
+// A[q][c], m columns, full column rank), the others 0 (synchronous).
+int virtual_state(Ctx &ctx, const void *state, int prec, unsigned n, unsigned m, const uint64_t *rows,
+                  const uint8_t *b, double fx, double fy, double *out);
 // One general pair sweep (any delta / selector).
 int u3_pair_apply(Ctx &ctx, void *state, int prec, unsigned nbits, const U3Gate &g);
 // The U3 of a qubit expansion: delta is the state's top bit (nbits - 1) and

@@ -1190,7 +1190,7 @@ int Sim::device_ptr(void **p, size_t *m) const
 
 // get_state (zxh.cpp:579-636): virt = A*real ^ b, stored at the bit-reversed
 // index, times the global phase.
-int Sim::get_state(double *out, size_t out_len) const
+int Sim::get_state(double *out, size_t out_len)
 {
     if (!executed_)
     {
@@ -1208,33 +1208,8 @@ int Sim::get_state(double *out, size_t out_len) const
         set_error("output buffer too small");
         return EINVAL_;
     }
-    const size_t real_size = size_t(1) << m_;
-    std::vector<std::complex<double>> real_state(real_size);
-    if (prec_ == C128)
-    {
-        ZXA_HIP(hipMemcpy(real_state.data(), dstate_, real_size * 16, hipMemcpyDeviceToHost));
-    }
-    else
-    {
-        std::vector<std::complex<float>> tmp(real_size);
-        ZXA_HIP(hipMemcpy(tmp.data(), dstate_, real_size * 8, hipMemcpyDeviceToHost));
-        for (size_t i = 0; i < real_size; i++)
-            real_state[i] = std::complex<double>(tmp[i].real(), tmp[i].imag());
-    }
-    std::fill(out, out + 2 * vsize, 0.0);
-    for (size_t real = 0; real < real_size; real++)
-    {
-        uint64_t virt = 0;
-        for (size_t q = 0; q < N_; q++)
-            virt |= uint64_t((__builtin_popcountll(real & rows_[q]) & 1) ^ b_[q]) << q;
-        uint64_t rev = 0;
-        for (size_t i = 0; i < N_; i++)
-            rev = (rev << 1) | ((virt >> i) & 1u);
-        const std::complex<double> v = real_state[real] * gphase_;
-        out[2 * rev] = v.real();
-        out[2 * rev + 1] = v.imag();
-    }
-    return OK;
+    return virtual_state(ctx_, dstate_, prec_, unsigned(N_), unsigned(m_), rows_.data(), b_.data(), gphase_.real(),
+                         gphase_.imag(), out);
 }
 
 } // namespace zxa

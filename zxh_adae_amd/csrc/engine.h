@@ -79,7 +79,7 @@ class Sim
     }
     int get_results(uint64_t *packed, size_t shots) const;
     int get_real_results(uint64_t *real, size_t shots) const;
-    int get_state(double *out, size_t out_len) const;
+    int get_state(double *out, size_t out_len);
     size_t required_M() const;
     size_t num_qubits() const
     {

@@ -4,6 +4,7 @@
 #include "dev.h"
 
 #include <algorithm>
+#include <vector>
 
 namespace zxa
 {
@@ -136,6 +137,50 @@ __global__ __launch_bounds__(kThreads) void gather_kernel(const void *__restrict
         static_cast<double2 *>(out)[i] = static_cast<const double2 *>(state)[idx[i]];
 }
 
+// out[i] = f psi[x] for output index first + i, x the address its virtual
+// index comes from, or 0 where it comes from none: w = w0 XOR the columns of
+// i's bits holds x in its low m bits and the checks of the affine map's image
+// above them.  Writes are contiguous and one to a thread; the reads follow
+// the map (bit-reversed for the plain method), 16 bytes each from the cache
+// level the state sits in, and stay far below the copy to the host that
+// follows.  The products round separately, as the host's did.
+struct MapCols
+{
+    uint64_t c[40];
+};
+template <bool kC64>
+__global__ __launch_bounds__(kThreads) void virtual_state_kernel(const void *__restrict__ state, unsigned m,
+                                                                 const MapCols cols, unsigned nbits, uint64_t w0,
+                                                                 double fx, double fy, double2 *__restrict__ out)
+{
+#pragma clang fp contract(off)
+    const uint64_t i = uint64_t(blockIdx.x) * kThreads + threadIdx.x;
+    if (i >> nbits)
+        return;
+    uint64_t w = w0;
+    for (unsigned k = 0; k < nbits; k++)
+        w ^= ((i >> k) & 1u) ? cols.c[k] : 0;
+    double2 r = make_double2(0.0, 0.0);
+    if ((w >> m) == 0)
+    {
+        double x, y;
+        if constexpr (kC64)
+        {
+            const float2 a = static_cast<const float2 *>(state)[w];
+            x = a.x;
+            y = a.y;
+        }
+        else
+        {
+            const double2 a = static_cast<const double2 *>(state)[w];
+            x = a.x;
+            y = a.y;
+        }
+        r = make_double2(x * fx - y * fy, x * fy + y * fx);
+    }
+    out[i] = r;
+}
+
 template <typename K>
 unsigned stream_grid(Ctx &ctx, K kernel, uint64_t n16)
 {
@@ -245,6 +290,79 @@ int gather(Ctx &ctx, const void *state, int prec, unsigned n, const uint64_t *id
     if (dout)
         (void)hipFree(dout);
     return hip_check(e, "gather");
+}
+
+int virtual_state(Ctx &ctx, const void *state, int prec, unsigned n, unsigned m, const uint64_t *rows,
+                  const uint8_t *b, double fx, double fy, double *out)
+{
+    // Gauss-Jordan on [A | I]: pivot row c becomes the combination of virtual
+    // bits that is address bit c, the other rows the combinations that vanish
+    // on the map's image
+    if (n >= 40 || m > n)
+    {
+        set_error("virtual state: needs fewer than 40 qubits and no more address bits than qubits");
+        return EINVAL_;
+    }
+    std::vector<uint64_t> a(rows, rows + n), t(n);
+    for (unsigned q = 0; q < n; q++)
+        t[q] = uint64_t(1) << q;
+    for (unsigned c = 0; c < m; c++)
+    {
+        unsigned p = c;
+        while (p < n && !((a[p] >> c) & 1u))
+            p++;
+        if (p == n)
+        {
+            set_error("virtual state: the affine map is not injective");
+            return EINVAL_;
+        }
+        std::swap(a[p], a[c]);
+        std::swap(t[p], t[c]);
+        for (unsigned k = 0; k < n; k++)
+            if (k != c && ((a[k] >> c) & 1u))
+            {
+                a[k] ^= a[c];
+                t[k] ^= t[c];
+            }
+    }
+    // the word of virtual bit q; output index bit n-1-q is virtual bit q
+    auto word = [&](unsigned q) {
+        uint64_t w = 0;
+        for (unsigned k = 0; k < n; k++)
+            w |= ((t[k] >> q) & 1u) << k;
+        return w;
+    };
+    uint64_t wb = 0;
+    MapCols cols = {};
+    for (unsigned q = 0; q < n; q++)
+    {
+        const uint64_t w = word(q);
+        cols.c[n - 1 - q] = w;
+        if (b[q])
+            wb ^= w;
+    }
+    const unsigned cbits = std::min(n, 22u); // 64 MiB of output at a time
+    const uint64_t chunk = uint64_t(1) << cbits;
+    ZXA_TRY(ctx.scratch_c.ensure(chunk * sizeof(double2)));
+    double2 *dev = static_cast<double2 *>(ctx.scratch_c.ptr);
+    const unsigned grid = unsigned((chunk + kThreads - 1) / kThreads);
+    for (uint64_t first = 0; first < (uint64_t(1) << n); first += chunk)
+    {
+        uint64_t w0 = wb;
+        for (unsigned k = cbits; k < n; k++)
+            if ((first >> k) & 1u)
+                w0 ^= cols.c[k];
+        if (prec == C64)
+            hipLaunchKernelGGL(virtual_state_kernel<true>, dim3(grid), dim3(kThreads), 0, ctx.stream, state, m, cols,
+                               cbits, w0, fx, fy, dev);
+        else
+            hipLaunchKernelGGL(virtual_state_kernel<false>, dim3(grid), dim3(kThreads), 0, ctx.stream, state, m, cols,
+                               cbits, w0, fx, fy, dev);
+        ZXA_HIP(hipGetLastError());
+        ZXA_HIP(hipMemcpyAsync(out + 2 * first, dev, chunk * sizeof(double2), hipMemcpyDeviceToHost, ctx.stream));
+    }
+    ZXA_HIP(hipStreamSynchronize(ctx.stream));
+    return OK;
 }
 
 int set_ones(Ctx &ctx, const uint64_t *dstates, int count, int prec)
