@@ -7,6 +7,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <random>
 #include <new>
 
 using zxa::Sim;
@@ -593,15 +594,8 @@ int zxh_k_sample(const void *state, int precision, size_t m, size_t seg_bits, ui
     if (shots == 0)
         return ZXH_OK;
     WITH_CTX(c);
-    double total = 0.0;
-    rc = zxa::sample_prepare(*c, state, precision, unsigned(m), unsigned(seg_bits), &total);
-    if (rc)
-        return rc;
-    if (!(total > 0.0))
-        return fail(ZXH_EZEROPROB, "state has zero total probability");
-    std::vector<double> thr(shots);
-    zxa::threshold_stream(stream_seed, shots, 0.0, total, thr.data());
-    return zxa::sample_search(*c, state, precision, thr.data(), shots, out_real);
+    return zxa::measure_affine(*c, state, precision, unsigned(m), unsigned(seg_bits), 0, nullptr, nullptr,
+                               stream_seed, shots, nullptr, out_real);
 }
 
 int zxh_k_measure(const void *state, int precision, size_t m, size_t seg_bits, size_t nq, const uint64_t *rows,
@@ -620,8 +614,9 @@ int zxh_k_measure(const void *state, int precision, size_t m, size_t seg_bits, s
     if (shots == 0)
         return ZXH_OK;
     WITH_CTX(c);
+    const uint64_t base = use_seed ? seed : uint64_t(std::random_device{}());
     return zxa::measure_affine(*c, state, precision, unsigned(m), unsigned(seg_bits), unsigned(nq), rows, b,
-                               use_seed != 0, seed, shots, packed, out_real);
+                               zxa::mix_seed(base, 0), shots, packed, out_real);
 }
 
 int zxh_k_sample_thresholds(const void *state, int precision, size_t m, size_t seg_bits, const double *thresholds,

@@ -86,9 +86,16 @@ int PinBuf::ensure(size_t need)
         return OK;
     release();
     const size_t cap = std::max<size_t>(need, 4096);
-    hipError_t e = hipHostMalloc(&ptr, cap, hipHostMallocDefault);
+    hipError_t e = hipHostMalloc(&ptr, cap, hipHostMallocMapped | hipHostMallocCoherent);
+    void *dev = nullptr;
+    if (e == hipSuccess)
+        e = hipHostGetDevicePointer(&dev, ptr, 0);
+    if (e == hipSuccess && dev != ptr)
+        e = hipErrorInvalidDevicePointer;
     if (e != hipSuccess)
     {
+        if (ptr)
+            (void)hipHostFree(ptr);
         ptr = nullptr;
         bytes = 0;
         set_error(std::string("hipHostMalloc failed: ") + hipGetErrorString(e));
@@ -437,7 +444,7 @@ void threshold_factors(double *uf, size_t cnt)
         th.join();
 }
 
-void threshold_apply(double *fh, size_t cnt, double begin, double end)
+double threshold_apply(double *fh, size_t cnt, double begin, double end)
 {
     double lo = begin;
     for (size_t k = 0; k < cnt; k++)
@@ -447,13 +454,7 @@ void threshold_apply(double *fh, size_t cnt, double begin, double end)
         fh[k] = head;
         lo = head;
     }
-}
-
-void threshold_stream(uint64_t stream_seed, size_t cnt, double begin, double end, double *out)
-{
-    threshold_draws(stream_seed, cnt, out);
-    threshold_factors(out, cnt);
-    threshold_apply(out, cnt, begin, end);
+    return lo;
 }
 
 } // namespace zxa

@@ -9,6 +9,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -73,7 +74,8 @@ struct DevBuf
     }
 };
 
-// Grow-only pinned host buffer (hipHostMalloc).
+// Grow-only pinned host buffer (hipHostMalloc; mapped and coherent, at the
+// same address for kernels).
 struct PinBuf
 {
     void *ptr = nullptr;
@@ -166,7 +168,7 @@ struct Ctx
     ParamRing ring;
     DevBuf scratch_a; // diag per-chunk coefficients
     DevBuf scratch_b; // sampler tree levels
-    DevBuf scratch_c; // sampler thresholds / results
+    DevBuf scratch_c; // sampler's rows (over 64 qubits); get_state output
     DevBuf scratch_d; // sampler per-segment tails
     DevBuf scratch_e; // observable per-workgroup partial sums
     DevBuf scratch_f; // adjoint per-wave transition accumulators
@@ -177,8 +179,9 @@ struct Ctx
     alignas(8) unsigned char sample_levels[64 * 8] = {};
     unsigned sample_m = 0, sample_I = 0;
     bool sample_ready = false;
-    PinBuf sample_total_pin; // the tree root, copied back asynchronously
-    PinBuf sample_thr_pin;   // thresholds of the kernel-level measure
+    PinBuf sample_total_pin; // the tree root and the search's error flag, written by the kernels
+    PinBuf sample_thr_pin;   // thresholds of the kernel-level sampler
+    PinBuf sample_out_pin;   // its results
     template <typename T>
     T &sample_levels_as()
     {
@@ -446,17 +449,14 @@ int state_reset(Ctx &ctx, void *state, int prec, size_t alloc_elems);
 int copy_apply(Ctx &ctx, void *dst, const void *src, size_t bytes);
 int scale_apply(Ctx &ctx, void *state, int prec, unsigned nbits, double re, double im);
 
-// Sampling in two steps: prepare builds the probability tree of 2^m
-// amplitudes and returns the total (the reference's local_prob); search
-// resolves sorted thresholds (host array) against it.
-int sample_prepare(Ctx &ctx, const void *state, int prec, unsigned m, unsigned seg_bits, double *total);
-// sample_prepare in two halves, so that host work can overlap the tree build:
-// launch enqueues it (and the copy of the root to pinned memory); total waits.
+// Sampling in two steps: launch enqueues the probability tree of 2^m
+// amplitudes (host work can overlap it), total waits for its root (the
+// reference's local_prob); search resolves sorted thresholds against it.
 int sample_launch(Ctx &ctx, const void *state, int prec, unsigned m, unsigned seg_bits);
 int sample_total(Ctx &ctx, double *total);
 // Optional packing of the samples into virtual result words on the device:
-// bit q = parity(real & rows[q]) ^ b[q]; out (host) gets ceil(nq / 64) words
-// per shot.
+// bit q = parity(real & rows[q]) ^ b[q]; out (pinned host memory) gets
+// ceil(nq / 64) words per shot.
 struct PackSpec
 {
     unsigned nq = 0;
@@ -464,16 +464,20 @@ struct PackSpec
     const uint8_t *b = nullptr;
     uint64_t *out = nullptr;
 };
-int sample_search(Ctx &ctx, const void *state, int prec, const double *thresholds, size_t shots, uint64_t *out_real,
-                  const PackSpec *pack = nullptr);
+// thr and real: pinned host memory (PinBuf), used in place by the kernel.
+// next (nullable) forms thresholds [from, to) just before they are searched.
+int sample_search(Ctx &ctx, const void *state, int prec, const double *thr, size_t shots, uint64_t *real,
+                  const PackSpec *pack, const std::function<void(size_t, size_t)> &next);
+// A whole draw from stream_seed: tree, thresholds (into thr) and search.
+int sample_draw(Ctx &ctx, const void *state, int prec, unsigned m, unsigned seg_bits, uint64_t stream_seed,
+                size_t shots, double *thr, uint64_t *real, const PackSpec *pack);
 // measure (measure_common.cpp:73-92) on a caller's state of 2^m amplitudes
-// and affine map (rows[q] bit c = A[q][c], b[q]; nq virtual qubits):
-// thresholds from mix_seed(use_seed ? seed : random_device, 0), segments of
-// 2^min(m, seg_bits); packed gets ceil(nq / 64) words per shot, out_real
-// (nullable) the real addresses, ascending.
+// and affine map (rows[q] bit c = A[q][c], b[q]; nq virtual qubits), segments
+// of 2^min(m, seg_bits); packed gets ceil(nq / 64) words per shot, out_real
+// (nullable) the real addresses, ascending.  nq = 0: real addresses only.
 int measure_affine(Ctx &ctx, const void *state, int prec, unsigned m, unsigned seg_bits, unsigned nq,
-                   const uint64_t *rows, const uint8_t *b, bool use_seed, uint64_t seed, size_t shots,
-                   uint64_t *packed, uint64_t *out_real);
+                   const uint64_t *rows, const uint8_t *b, uint64_t stream_seed, size_t shots, uint64_t *packed,
+                   uint64_t *out_real);
 // Both steps with caller-given thresholds.
 int sample_apply(Ctx &ctx, const void *state, int prec, unsigned m, unsigned seg_bits, const double *thresholds,
                  size_t shots, uint64_t *out_real);
@@ -492,16 +496,16 @@ int observable_apply(Ctx &ctx, const void *src, void *dst, int prec, unsigned nb
 // and max_i |a_i - b_i|.
 int compare_states(Ctx &ctx, const void *a, int prec_a, const void *b, int prec_b, unsigned n, double *out5);
 
-// Host threshold stream (measure_common.cpp:14-71) from an already mixed seed.
-void threshold_stream(uint64_t stream_seed, size_t cnt, double begin, double end, double *out);
-// The same stream in three steps.  draws: the cnt uniforms u_k (mt19937_64,
+// Host threshold stream (measure_common.cpp:14-71) from an already mixed seed,
+// in three steps.  draws: the cnt uniforms u_k (mt19937_64,
 // uniform_real_distribution, clamped below by DBL_MIN), in order.  factors:
 // in place, f_k = 1 - u_k^(1 / (cnt - k)), which does not depend on the
 // interval, on host threads.  apply: in place, the recurrence
-// head_k = lo + (end - lo) * f_k, lo = head_k, from lo = begin.
+// head_k = lo + (end - lo) * f_k, lo = head_k, from lo = begin; returns the
+// last head, so that it can go on from there.
 void threshold_draws(uint64_t stream_seed, size_t cnt, double *u);
 void threshold_factors(double *uf, size_t cnt);
-void threshold_apply(double *fh, size_t cnt, double begin, double end);
+double threshold_apply(double *fh, size_t cnt, double begin, double end);
 uint64_t mix_seed(uint64_t base, uint64_t salt);
 
 } // namespace zxa

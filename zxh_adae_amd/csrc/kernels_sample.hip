@@ -23,7 +23,7 @@
 
 #include <algorithm>
 #include <cstring>
-#include <random>
+#include <functional>
 #include <vector>
 
 #pragma clang fp contract(off)
@@ -57,11 +57,23 @@ __device__ __forceinline__ double p_of(const void *state, bool c64, uint64_t i)
 // One workgroup reduces up to 2^kSpanBits input values of level lin into the
 // levels lin+1 .. lin+span_bits and stores every level in [LS, m] it owns.
 // src_kind: 0 = c128 amplitudes, 1 = c64 amplitudes, 2 = tree nodes (f64).
+// The root (level m) also goes to root[0] (host memory), and, when one segment
+// is the whole state, to one[0..1] as that segment's prefix (0) and tail.
 __global__ __launch_bounds__(kThreads) void tree_kernel(const void *__restrict__ src, int src_kind, int lin,
                                                         int span_bits, int LS, int m, double *__restrict__ tree,
-                                                        const Levels lv)
+                                                        const Levels lv, double *__restrict__ root,
+                                                        double *__restrict__ one)
 {
     __shared__ double buf[1 << kSpanBits];
+    auto top = [&](double v) {
+        if (root)
+            root[0] = v;
+        if (one)
+        {
+            one[0] = 0.0;
+            one[1] = __dadd_rn(0.0, v);
+        }
+    };
     const int span = 1 << span_bits;
     const uint64_t g0 = static_cast<uint64_t>(blockIdx.x) << span_bits;
     for (int i = threadIdx.x; i < span; i += kThreads)
@@ -74,6 +86,8 @@ __global__ __launch_bounds__(kThreads) void tree_kernel(const void *__restrict__
         buf[i] = v;
         if (src_kind != 2 && lin >= LS)
             tree[lv.off[lin] + g0 + i] = v;
+        if (lin == m)
+            top(v);
     }
     __syncthreads();
     for (int r = 1; r <= span_bits; r++)
@@ -92,6 +106,8 @@ __global__ __launch_bounds__(kThreads) void tree_kernel(const void *__restrict__
             buf[k] = v;
             if (l >= LS && l <= m)
                 tree[lv.off[l] + (g0 >> r) + k] = v;
+            if (l == m)
+                top(v);
         }
         __syncthreads();
     }
@@ -320,67 +336,91 @@ __global__ __launch_bounds__(kThreads) void cummax_kernel(double *__restrict__ v
     }
 }
 
-template <int N>
-__device__ __forceinline__ double pick(const double (&a)[N], int idx)
+// tails_kernel and cummax_kernel in one workgroup, for states of few
+// segments: each thread's run of segments, then the running maximum across the
+// threads by doubling (max is exact, so the order does not matter).
+constexpr int kFewThreads = 1024;
+constexpr uint64_t kFewSegs = 4096;
+__global__ __launch_bounds__(kFewThreads) void few_tails_kernel(const double *__restrict__ tree, const Levels lv,
+                                                                int I, int m, int nseg, double *__restrict__ prefix,
+                                                                double *__restrict__ cmax)
 {
-    double r = 0.0;
+    __shared__ double part[kFewThreads];
+    constexpr int kPer = int(kFewSegs) / kFewThreads;
+    double t[kPer];
+    double mx = -1.0;
 #pragma unroll
-    for (int i = 0; i < N; i++)
-        r = (i == idx) ? a[i] : r;
-    return r;
+    for (int j = 0; j < kPer; j++)
+    {
+        const int s = int(threadIdx.x) * kPer + j;
+        t[j] = -1.0;
+        if (s < nseg)
+        {
+            double acc = 0.0;
+            for (int l = m - I - 1; l >= 0; l--)
+                if ((s >> l) & 1)
+                    acc = __dadd_rn(acc, tree[lv.off[I + l] + uint64_t((s >> l) - 1)]);
+            prefix[s] = acc;
+            t[j] = __dadd_rn(acc, tree[lv.off[I] + uint64_t(s)]);
+        }
+        mx = fmax(mx, t[j]);
+    }
+    part[threadIdx.x] = mx;
+    __syncthreads();
+    for (int d = 1; d < kFewThreads; d <<= 1)
+    {
+        const double o = int(threadIdx.x) >= d ? part[threadIdx.x - d] : -1.0;
+        __syncthreads();
+        part[threadIdx.x] = fmax(part[threadIdx.x], o);
+        __syncthreads();
+    }
+    double run = threadIdx.x ? part[threadIdx.x - 1] : -1.0;
+#pragma unroll
+    for (int j = 0; j < kPer; j++)
+    {
+        const int s = int(threadIdx.x) * kPer + j;
+        run = fmax(run, t[j]);
+        if (s < nseg)
+            cmax[s] = run;
+    }
 }
 
-// Levels below LB (<= kLBM) of the 2^LB-amplitude block holding g, as the
-// block's balanced pair sums: the Fenwick part of the exclusive prefix of g's
-// offset in the block (levels LB-1 .. 0, high to low) and p_g.
-template <int kLBM>
-__device__ __forceinline__ void block_prefix(const void *state, bool c64, uint64_t g, int LB, double &acc,
-                                             double &pg)
+// Virtual bits of a real address (pack_virtual_results_host,
+// src/zxh/src/measure/measure_result_pack.h:24-44; the reference's GPU path
+// does the same in map_real_to_virtual_words_kernel): virtual bit q = parity
+// (real & row q) ^ b[q], the row's bit 63 holding b[q].  Up to 64 rows travel
+// in the kernel arguments; more come from device memory.
+constexpr int kArgRows = 64;
+struct PackArgs
 {
-    constexpr int NB = 1 << kLBM;
-    const uint64_t gb = g & ~((uint64_t(1) << LB) - 1);
-    const int nb = 1 << LB;
-    double lv0[NB], lv1[NB / 2], lv2[NB / 4], lv3[NB / 8], lv4[NB / 16 > 0 ? NB / 16 : 1];
-#pragma unroll
-    for (int i = 0; i < NB; i++)
-        lv0[i] = i < nb ? p_of(state, c64, gb + i) : 0.0;
-#pragma unroll
-    for (int i = 0; i < NB / 2; i++)
-        lv1[i] = __dadd_rn(lv0[2 * i], lv0[2 * i + 1]);
-#pragma unroll
-    for (int i = 0; i < NB / 4; i++)
-        lv2[i] = __dadd_rn(lv1[2 * i], lv1[2 * i + 1]);
-#pragma unroll
-    for (int i = 0; i < NB / 8; i++)
-        lv3[i] = __dadd_rn(lv2[2 * i], lv2[2 * i + 1]);
-    if (kLBM == 5)
-    {
-#pragma unroll
-        for (int i = 0; i < NB / 16; i++)
-            lv4[i] = __dadd_rn(lv3[2 * i], lv3[2 * i + 1]);
-    }
-    const int off = static_cast<int>(g - gb);
-    if (kLBM == 5 && (off & 16))
-        acc = __dadd_rn(acc, lv4[0]);
-    if (off & 8)
-        acc = __dadd_rn(acc, pick(lv3, (off >> 3) - 1));
-    if (off & 4)
-        acc = __dadd_rn(acc, pick(lv2, (off >> 2) - 1));
-    if (off & 2)
-        acc = __dadd_rn(acc, pick(lv1, (off >> 1) - 1));
-    if (off & 1)
-        acc = __dadd_rn(acc, pick(lv0, off - 1));
-    pg = pick(lv0, off);
-}
+    uint64_t rows[kArgRows];
+    const uint64_t *more; // all nq rows when nq > kArgRows
+    uint64_t *out;        // nullptr: no packing
+    int nq, wc;
+};
 
 // One shot per thread.
+//
+// The probes of libstdc++'s upper_bound over a segment's 2^I values are
+// the midpoints of aligned blocks: after a right turn at mid the range is
+// (mid, end of mid's block), 2^l - 1 values whose own midpoint is again the
+// block's, and before the first right turn it is the block from 0.  So the
+// walk is a descent: at block [P, P + 2^l) the probe is mid = P + 2^(l-1),
+// whose prefix is that of P (carried, the same sums in the same order) plus
+// one stored node, the left half's.  A probe loads that node and the
+// amplitude at mid, both at once.  The last LB levels lie in one block of
+// 256 bytes, read once; its pair sums come from registers.  (Re-reading every
+// prefix node and a 256-byte block at each probe, 10^6 shots of a 30-qubit
+// complex128 state took 1.88 ms, and 1024 shots of a 20-qubit one 82 us of
+// dependent loads.)
 template <bool kC64>
 __global__ __launch_bounds__(kThreads) void search_kernel(const void *__restrict__ state,
                                                           const double *__restrict__ tree, const Levels lv, int I,
                                                           int LS, const double *__restrict__ cmax,
                                                           const double *__restrict__ prefix, uint64_t nseg,
                                                           const double *__restrict__ thr, uint64_t shots,
-                                                          uint64_t *__restrict__ out, int *__restrict__ err)
+                                                          uint64_t *__restrict__ out, int *__restrict__ err,
+                                                          const PackArgs pack)
 {
     const uint64_t k = blockIdx.x * static_cast<uint64_t>(blockDim.x) + threadIdx.x;
     if (k >= shots)
@@ -402,7 +442,6 @@ __global__ __launch_bounds__(kThreads) void search_kernel(const void *__restrict
     if (lo >= nseg)
     {
         *err = 1;
-        out[k] = 0;
         return;
     }
     const uint64_t seg = lo;
@@ -411,30 +450,68 @@ __global__ __launch_bounds__(kThreads) void search_kernel(const void *__restrict
     const int LB = LS < I ? LS : I; // low levels recomputed from amplitudes
     const uint64_t valid = uint64_t(1) << I;
 
-    // libstdc++ upper_bound probe sequence over cdf[0, valid)
-    uint64_t first = 0;
-    len = valid;
-    while (len > 0)
+    uint64_t P = 0;
+    double acc = 0.0;
+    for (int l = I; l > LB; l--)
     {
-        const uint64_t half = len >> 1;
-        const uint64_t mid = first + half;
-        const uint64_t g = sbase + mid;
-        double acc = 0.0;
-        for (int l = I - 1; l >= LB; l--)
-            if ((mid >> l) & 1u)
-                acc = __dadd_rn(acc, tree[lv.off[l] + ((g >> l) - 1)]);
-        double pmid;
-        block_prefix<kC64 ? 5 : 4>(state, kC64, g, LB, acc, pmid);
-        const double cdf = __dadd_rn(__dadd_rn(head, acc), pmid);
-        if (tau < cdf)
-            len = half;
-        else
+        const uint64_t mid = P + (uint64_t(1) << (l - 1));
+        const double left = tree[lv.off[l - 1] + ((sbase + P) >> (l - 1))];
+        const double pm = p_of(state, kC64, sbase + mid);
+        const double excl = __dadd_rn(acc, left);
+        if (!(tau < __dadd_rn(__dadd_rn(head, excl), pm)))
         {
-            first = mid + 1;
-            len = len - half - 1;
+            P = mid;
+            acc = excl;
         }
     }
-    out[k] = sbase + (first == valid ? valid - 1 : first);
+    // the block of 2^LB amplitudes from P on and its aligned pair sums; a turn
+    // halves the window they cover, which stays at the arrays' front
+    constexpr int kLBM = kC64 ? 5 : 4;
+    constexpr int NB = 1 << kLBM;
+    double q[kLBM][NB];
+#pragma unroll
+    for (int i = 0; i < NB; i++)
+        q[0][i] = i < (1 << LB) ? p_of(state, kC64, sbase + P + i) : 0.0;
+#pragma unroll
+    for (int r = 1; r < kLBM; r++)
+#pragma unroll
+        for (int i = 0; i < (NB >> r); i++)
+            q[r][i] = __dadd_rn(q[r - 1][2 * i], q[r - 1][2 * i + 1]);
+    const double p0 = q[0][0];
+#pragma unroll
+    for (int l = kLBM; l > 0; l--)
+    {
+        if (l > LB)
+            continue;
+        const int half = 1 << (l - 1);
+        const double excl = __dadd_rn(acc, q[l - 1][0]);
+        const bool right = !(tau < __dadd_rn(__dadd_rn(head, excl), q[0][half]));
+        P = right ? P + half : P;
+        acc = right ? excl : acc;
+#pragma unroll
+        for (int r = 0; r < l - 1; r++)
+#pragma unroll
+            for (int i = 0; i < (half >> r); i++)
+                q[r][i] = right ? q[r][i + (half >> r)] : q[r][i];
+    }
+    // without a right turn value 0 is still to be probed
+    uint64_t first = P + 1;
+    if (P == 0 && tau < __dadd_rn(__dadd_rn(head, 0.0), p0))
+        first = 0;
+    const uint64_t real = sbase + (first == valid ? valid - 1 : first);
+    out[k] = real;
+    if (pack.out)
+        for (int w = 0; w < pack.wc; w++)
+        {
+            uint64_t word = 0;
+            const int hi = min(64, pack.nq - 64 * w);
+            for (int j = 0; j < hi; j++)
+            {
+                const uint64_t row = pack.more ? pack.more[64 * w + j] : pack.rows[j];
+                word |= uint64_t((__popcll(real & row & ~(uint64_t(1) << 63)) & 1) ^ int(row >> 63)) << j;
+            }
+            pack.out[k * uint64_t(pack.wc) + w] = word;
+        }
 }
 
 // Lowest stored tree level: below it the search recomputes from amplitudes
@@ -444,7 +521,8 @@ inline unsigned low_level(int prec, unsigned I)
     return std::min(prec == C64 ? 5u : 4u, I);
 }
 
-int build_tree(Ctx &ctx, const void *state, int prec, unsigned m, unsigned LS, Levels &lv, double **tree_out)
+int build_tree(Ctx &ctx, const void *state, int prec, unsigned m, unsigned LS, Levels &lv, double **tree_out,
+               double *root, double *one)
 {
     uint64_t total = 0;
     for (unsigned l = 0; l < kMaxLevels; l++)
@@ -498,7 +576,7 @@ int build_tree(Ctx &ctx, const void *state, int prec, unsigned m, unsigned LS, L
             return EINVAL_;
         }
         hipLaunchKernelGGL(tree_kernel, dim3(static_cast<unsigned>(groups)), dim3(kThreads), 0, ctx.stream, src, kind,
-                           lin, span_bits, int(LS), int(m), tree, lv);
+                           lin, span_bits, int(LS), int(m), tree, lv, root, one);
         ZXA_HIP(hipGetLastError());
         first = false;
         lin += span_bits;
@@ -514,14 +592,31 @@ int build_tree(Ctx &ctx, const void *state, int prec, unsigned m, unsigned LS, L
 
 } // namespace
 
+// What the sampler's kernels tell the host: in pinned, coherent memory.
+struct Told
+{
+    double total;
+    int err;
+};
+
+int told(Ctx &ctx, Told **t)
+{
+    ZXA_TRY(ctx.sample_total_pin.ensure(sizeof(Told)));
+    *t = static_cast<Told *>(ctx.sample_total_pin.ptr);
+    return OK;
+}
+
 int prob_total(Ctx &ctx, const void *state, int prec, unsigned m, double *out)
 {
     Levels lv;
     double *tree = nullptr;
+    Told *t = nullptr;
+    ZXA_TRY(told(ctx, &t));
     const unsigned LS = low_level(prec, m);
-    ZXA_TRY(build_tree(ctx, state, prec, m, LS, lv, &tree));
-    ZXA_HIP(hipMemcpyAsync(out, tree + lv.off[m], sizeof(double), hipMemcpyDeviceToHost, ctx.stream));
+    ctx.sample_ready = false; // the tree of a launch before this one is overwritten
+    ZXA_TRY(build_tree(ctx, state, prec, m, LS, lv, &tree, &t->total, nullptr));
     ZXA_HIP(hipStreamSynchronize(ctx.stream));
+    *out = t->total;
     return OK;
 }
 
@@ -537,19 +632,27 @@ int sample_launch(Ctx &ctx, const void *state, int prec, unsigned m, unsigned se
     const unsigned LS = low_level(prec, I);
     Levels &lv = ctx.sample_levels_as<Levels>();
     double *tree = nullptr;
-    ZXA_TRY(ctx.sample_total_pin.ensure(sizeof(double)));
-    ZXA_TRY(build_tree(ctx, state, prec, m, LS, lv, &tree));
+    Told *t = nullptr;
+    ZXA_TRY(told(ctx, &t));
     const uint64_t nseg = uint64_t(1) << (m - I);
     ZXA_TRY(ctx.scratch_d.ensure(2 * nseg * sizeof(double)));
     double *prefix = static_cast<double *>(ctx.scratch_d.ptr);
     double *cmax = prefix + nseg;
-    hipLaunchKernelGGL(tails_kernel, dim3(static_cast<unsigned>((nseg + kThreads - 1) / kThreads)), dim3(kThreads), 0,
-                       ctx.stream, tree, lv, int(I), int(m), nseg, prefix, cmax);
-    ZXA_HIP(hipGetLastError());
-    hipLaunchKernelGGL(cummax_kernel, dim3(1), dim3(kThreads), 0, ctx.stream, cmax, nseg);
-    ZXA_HIP(hipGetLastError());
-    ZXA_HIP(hipMemcpyAsync(ctx.sample_total_pin.ptr, tree + lv.off[m], sizeof(double), hipMemcpyDeviceToHost,
-                           ctx.stream));
+    ZXA_TRY(build_tree(ctx, state, prec, m, LS, lv, &tree, &t->total, nseg == 1 ? prefix : nullptr));
+    if (nseg > kFewSegs)
+    {
+        hipLaunchKernelGGL(tails_kernel, dim3(static_cast<unsigned>((nseg + kThreads - 1) / kThreads)),
+                           dim3(kThreads), 0, ctx.stream, tree, lv, int(I), int(m), nseg, prefix, cmax);
+        ZXA_HIP(hipGetLastError());
+        hipLaunchKernelGGL(cummax_kernel, dim3(1), dim3(kThreads), 0, ctx.stream, cmax, nseg);
+        ZXA_HIP(hipGetLastError());
+    }
+    else if (nseg > 1)
+    {
+        hipLaunchKernelGGL(few_tails_kernel, dim3(1), dim3(kFewThreads), 0, ctx.stream, tree, lv, int(I), int(m),
+                           int(nseg), prefix, cmax);
+        ZXA_HIP(hipGetLastError());
+    }
     ctx.sample_m = m;
     ctx.sample_I = I;
     ctx.sample_ready = true;
@@ -564,7 +667,7 @@ int sample_total(Ctx &ctx, double *total)
         return ESTATE;
     }
     ZXA_HIP(hipStreamSynchronize(ctx.stream));
-    *total = *static_cast<const double *>(ctx.sample_total_pin.ptr);
+    *total = static_cast<const Told *>(ctx.sample_total_pin.ptr)->total;
     return OK;
 }
 
@@ -574,34 +677,12 @@ int sample_prepare(Ctx &ctx, const void *state, int prec, unsigned m, unsigned s
     return sample_total(ctx, total);
 }
 
-// Real address -> virtual result words (pack_virtual_results_host,
-// src/zxh/src/measure/measure_result_pack.h:24-44; the reference's GPU path
-// does the same in map_real_to_virtual_words_kernel): virtual bit q of shot i
-// = parity(real[i] & rows[q]) ^ b[q], packed into wc 64-bit words per shot.
-__global__ __launch_bounds__(kThreads) void pack_kernel(const uint64_t *__restrict__ real, uint64_t shots,
-                                                        const uint64_t *__restrict__ rows,
-                                                        const uint8_t *__restrict__ b, int nq, int wc,
-                                                        uint64_t *__restrict__ out)
-{
-    const uint64_t i = uint64_t(blockIdx.x) * kThreads + threadIdx.x;
-    if (i >= shots)
-        return;
-    const uint64_t r = real[i];
-    for (int w = 0; w < wc; w++)
-    {
-        uint64_t word = 0;
-        const int hi = min(64, nq - 64 * w);
-        for (int k = 0; k < hi; k++)
-        {
-            const int q = 64 * w + k;
-            word |= uint64_t((__popcll(r & rows[q]) & 1) ^ b[q]) << k;
-        }
-        out[i * uint64_t(wc) + w] = word;
-    }
-}
-
-int sample_search(Ctx &ctx, const void *state, int prec, const double *thresholds, size_t shots, uint64_t *out_real,
-                  const PackSpec *pack)
+// Resolves the thresholds of a sampler launch.  thr, real and pack->out are
+// pinned host memory (the kernel reads and writes them in place); next, when
+// given, forms thresholds [from, to) just before they are searched, so that
+// the search of one piece runs while the host forms the next.
+int sample_search(Ctx &ctx, const void *state, int prec, const double *thr, size_t shots, uint64_t *real,
+                  const PackSpec *pack, const std::function<void(size_t, size_t)> &next)
 {
     if (shots == 0)
         return OK;
@@ -617,44 +698,52 @@ int sample_search(Ctx &ctx, const void *state, int prec, const double *threshold
     const uint64_t nseg = uint64_t(1) << (m - I);
     const double *prefix = static_cast<const double *>(ctx.scratch_d.ptr);
     const double *cmax = prefix + nseg;
-    const size_t wc = pack ? (size_t(pack->nq) + 63) / 64 : 0;
-    const size_t nq = pack ? pack->nq : 0;
-    // thresholds | real results | packed words | rows | error flag | b
-    const size_t need = shots * (sizeof(double) + sizeof(uint64_t) * (1 + wc)) + nq * sizeof(uint64_t) + 64 + nq;
-    ZXA_TRY(ctx.scratch_c.ensure(need));
-    double *dthr = static_cast<double *>(ctx.scratch_c.ptr);
-    uint64_t *dout = reinterpret_cast<uint64_t *>(dthr + shots);
-    uint64_t *dpacked = dout + shots;
-    uint64_t *drows = dpacked + shots * wc;
-    int *derr = reinterpret_cast<int *>(drows + nq);
-    uint8_t *db = reinterpret_cast<uint8_t *>(derr + 16);
-    ZXA_HIP(hipMemcpyAsync(dthr, thresholds, shots * sizeof(double), hipMemcpyHostToDevice, ctx.stream));
-    ZXA_HIP(hipMemsetAsync(derr, 0, sizeof(int), ctx.stream));
-    const unsigned grid = static_cast<unsigned>((shots + kThreads - 1) / kThreads);
-    ZXA_TRY(ctx.tic());
-    if (prec == C64)
-        hipLaunchKernelGGL(search_kernel<true>, dim3(grid), dim3(kThreads), 0, ctx.stream, state, tree, lv, int(I),
-                           int(LS), cmax, prefix, nseg, dthr, uint64_t(shots), dout, derr);
-    else
-        hipLaunchKernelGGL(search_kernel<false>, dim3(grid), dim3(kThreads), 0, ctx.stream, state, tree, lv, int(I),
-                           int(LS), cmax, prefix, nseg, dthr, uint64_t(shots), dout, derr);
-    ZXA_HIP(hipGetLastError());
-    ZXA_TRY(ctx.toc(F_SAMPLE, 0));
+    Told *t = nullptr;
+    ZXA_TRY(told(ctx, &t));
+    t->err = 0;
+    PackArgs pa = {};
+    std::vector<uint64_t> rows;
     if (pack)
     {
-        ZXA_HIP(hipMemcpyAsync(drows, pack->rows, nq * sizeof(uint64_t), hipMemcpyHostToDevice, ctx.stream));
-        ZXA_HIP(hipMemcpyAsync(db, pack->b, nq, hipMemcpyHostToDevice, ctx.stream));
-        hipLaunchKernelGGL(pack_kernel, dim3(grid), dim3(kThreads), 0, ctx.stream, dout, uint64_t(shots), drows, db,
-                           int(nq), int(wc), dpacked);
-        ZXA_HIP(hipGetLastError());
-        ZXA_HIP(hipMemcpyAsync(pack->out, dpacked, shots * wc * sizeof(uint64_t), hipMemcpyDeviceToHost,
-                               ctx.stream));
+        pa.nq = int(pack->nq);
+        pa.wc = (pa.nq + 63) / 64;
+        rows.resize(size_t(pa.nq));
+        for (int q = 0; q < pa.nq; q++)
+            rows[size_t(q)] = pack->rows[q] | (uint64_t(pack->b[q] & 1u) << 63);
+        if (pa.nq <= kArgRows)
+            std::copy(rows.begin(), rows.end(), pa.rows);
+        else
+        {
+            ZXA_TRY(ctx.scratch_c.ensure(rows.size() * sizeof(uint64_t)));
+            ZXA_HIP(hipMemcpyAsync(ctx.scratch_c.ptr, rows.data(), rows.size() * sizeof(uint64_t),
+                                   hipMemcpyHostToDevice, ctx.stream));
+            pa.more = static_cast<const uint64_t *>(ctx.scratch_c.ptr);
+        }
     }
-    int herr = 0;
-    ZXA_HIP(hipMemcpyAsync(out_real, dout, shots * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx.stream));
-    ZXA_HIP(hipMemcpyAsync(&herr, derr, sizeof(int), hipMemcpyDeviceToHost, ctx.stream));
+    // pieces of 128 K shots: 0.2 ms of threshold recurrence each, several
+    // times what the search of one takes, so only the last is not hidden
+    constexpr size_t kPiece = size_t(1) << 17;
+    ZXA_TRY(ctx.tic());
+    for (size_t o = 0; o < shots; o += kPiece)
+    {
+        const size_t cnt = next ? std::min(kPiece, shots - o) : shots;
+        if (next)
+            next(o, o + cnt);
+        pa.out = pack ? pack->out + o * size_t(pa.wc) : nullptr;
+        const unsigned grid = static_cast<unsigned>((cnt + kThreads - 1) / kThreads);
+        if (prec == C64)
+            hipLaunchKernelGGL(search_kernel<true>, dim3(grid), dim3(kThreads), 0, ctx.stream, state, tree, lv,
+                               int(I), int(LS), cmax, prefix, nseg, thr + o, uint64_t(cnt), real + o, &t->err, pa);
+        else
+            hipLaunchKernelGGL(search_kernel<false>, dim3(grid), dim3(kThreads), 0, ctx.stream, state, tree, lv,
+                               int(I), int(LS), cmax, prefix, nseg, thr + o, uint64_t(cnt), real + o, &t->err, pa);
+        ZXA_HIP(hipGetLastError());
+        if (!next)
+            break;
+    }
+    ZXA_TRY(ctx.toc(F_SAMPLE, 0));
     ZXA_HIP(hipStreamSynchronize(ctx.stream));
-    if (herr)
+    if (t->err)
     {
         set_error("measure failed to resolve all local samples");
         return EUNRESOLVED;
@@ -662,21 +751,14 @@ int sample_search(Ctx &ctx, const void *state, int prec, const double *threshold
     return OK;
 }
 
-// measure (measure_common.cpp:73-92) on a caller's state and affine map:
-// the tree builds while the host draws the threshold stream's uniforms and
-// factors, the search resolves the thresholds, and the device packs the
-// virtual result words.
-int measure_affine(Ctx &ctx, const void *state, int prec, unsigned m, unsigned seg_bits, unsigned nq,
-                   const uint64_t *rows, const uint8_t *b, bool use_seed, uint64_t seed, size_t shots,
-                   uint64_t *packed, uint64_t *out_real)
+// The whole draw: the tree builds while the host forms the uniforms'
+// factors, which do not depend on the total; then the recurrence, piece by
+// piece ahead of the search.
+int sample_draw(Ctx &ctx, const void *state, int prec, unsigned m, unsigned seg_bits, uint64_t stream_seed,
+                size_t shots, double *thr, uint64_t *real, const PackSpec *pack)
 {
-    if (shots == 0)
-        return OK;
-    ZXA_TRY(sample_launch(ctx, state, prec, m, std::min(m, seg_bits)));
-    const uint64_t base = use_seed ? seed : uint64_t(std::random_device{}());
-    ZXA_TRY(ctx.sample_thr_pin.ensure(shots * sizeof(double)));
-    double *thr = static_cast<double *>(ctx.sample_thr_pin.ptr);
-    threshold_draws(mix_seed(base, 0), shots, thr);
+    ZXA_TRY(sample_launch(ctx, state, prec, m, seg_bits));
+    threshold_draws(stream_seed, shots, thr);
     threshold_factors(thr, shots);
     double total = 0.0;
     ZXA_TRY(sample_total(ctx, &total));
@@ -685,19 +767,35 @@ int measure_affine(Ctx &ctx, const void *state, int prec, unsigned m, unsigned s
         set_error("state has zero total probability");
         return EZEROPROB;
     }
-    threshold_apply(thr, shots, 0.0, total);
-    std::vector<uint64_t> realv;
-    if (!out_real)
-    {
-        realv.resize(shots);
-        out_real = realv.data();
-    }
+    double lo = 0.0;
+    return sample_search(ctx, state, prec, thr, shots, real, pack,
+                         [&](size_t b, size_t e) { lo = threshold_apply(thr + b, e - b, lo, total); });
+}
+
+// measure (measure_common.cpp:73-92) on a caller's state and affine map;
+// nq = 0: real addresses only.
+int measure_affine(Ctx &ctx, const void *state, int prec, unsigned m, unsigned seg_bits, unsigned nq,
+                   const uint64_t *rows, const uint8_t *b, uint64_t stream_seed, size_t shots, uint64_t *packed,
+                   uint64_t *out_real)
+{
+    if (shots == 0)
+        return OK;
+    const size_t wc = (size_t(nq) + 63) / 64;
+    ZXA_TRY(ctx.sample_thr_pin.ensure(shots * sizeof(double)));
+    ZXA_TRY(ctx.sample_out_pin.ensure(shots * (1 + wc) * sizeof(uint64_t)));
+    uint64_t *real = static_cast<uint64_t *>(ctx.sample_out_pin.ptr);
     PackSpec ps;
     ps.nq = nq;
     ps.rows = rows;
     ps.b = b;
-    ps.out = packed;
-    return sample_search(ctx, state, prec, thr, shots, out_real, &ps);
+    ps.out = real + shots;
+    ZXA_TRY(sample_draw(ctx, state, prec, m, seg_bits, stream_seed, shots,
+                        static_cast<double *>(ctx.sample_thr_pin.ptr), real, nq ? &ps : nullptr));
+    if (nq)
+        std::memcpy(packed, ps.out, shots * wc * sizeof(uint64_t));
+    if (out_real)
+        std::memcpy(out_real, real, shots * sizeof(uint64_t));
+    return OK;
 }
 
 int sample_apply(Ctx &ctx, const void *state, int prec, unsigned m, unsigned seg_bits, const double *thresholds,
@@ -705,9 +803,16 @@ int sample_apply(Ctx &ctx, const void *state, int prec, unsigned m, unsigned seg
 {
     if (shots == 0)
         return OK;
+    ZXA_TRY(ctx.sample_thr_pin.ensure(shots * sizeof(double)));
+    ZXA_TRY(ctx.sample_out_pin.ensure(shots * sizeof(uint64_t)));
+    std::memcpy(ctx.sample_thr_pin.ptr, thresholds, shots * sizeof(double));
+    ZXA_TRY(sample_launch(ctx, state, prec, m, seg_bits));
     double total = 0.0;
-    ZXA_TRY(sample_prepare(ctx, state, prec, m, seg_bits, &total));
-    return sample_search(ctx, state, prec, thresholds, shots, out_real);
+    ZXA_TRY(sample_total(ctx, &total));
+    ZXA_TRY(sample_search(ctx, state, prec, static_cast<const double *>(ctx.sample_thr_pin.ptr), shots,
+                          static_cast<uint64_t *>(ctx.sample_out_pin.ptr), nullptr, nullptr));
+    std::memcpy(out_real, ctx.sample_out_pin.ptr, shots * sizeof(uint64_t));
+    return OK;
 }
 
 } // namespace zxa
