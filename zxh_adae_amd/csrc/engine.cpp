@@ -672,6 +672,24 @@ int Sim::emit_u3(std::vector<U3Gate> &descs)
     return OK;
 }
 
+void Sim::Acc::merge()
+{
+    if (!held)
+        return;
+    if (active)
+    {
+        const std::complex<double> a00 = u00, a01 = u01, a10 = u10, a11 = u11;
+        u00 = a00 * h00 + a01 * h10;
+        u01 = a00 * h01 + a01 * h11;
+        u10 = a10 * h00 + a11 * h10;
+        u11 = a10 * h01 + a11 * h11;
+    }
+    else
+        u00 = h00, u01 = h01, u10 = h10, u11 = h11;
+    held = false;
+    active = true;
+}
+
 // flush_u3_batch (zxh.cpp:390-428): one descriptor per active accumulator,
 // in qubit order; the batch is applied as tile passes.
 int Sim::flush_u3(std::vector<Acc> &pend, size_t &count)
@@ -683,6 +701,7 @@ int Sim::flush_u3(std::vector<Acc> &pend, size_t &count)
     for (size_t q = 0; q < N_; q++)
     {
         Acc &a = pend[q];
+        a.merge();
         if (!a.active)
             continue;
         U3Gate g;
@@ -763,12 +782,18 @@ int Sim::execute()
     //    (selector . delta = 0 over GF(2)), else post;
     //  - a U3 gate joins the batch when it commutes with every gate in post
     //    and every member of another run (alpha . delta' = alpha' . delta = 0),
-    //    or continues its own run's product on its qubit.  Otherwise pre and
+    //    continues its own run's product on its qubit, or follows an earlier
+    //    run's product there under the same descriptor.  Otherwise pre and
     //    the members of earlier runs are applied, and post becomes pre (no
     //    diagonal gate arrives inside a run, so the current run's members
     //    follow post in the circuit and commute with it).
     // Each run keeps its own product per qubit, as the reference forms it,
-    // so the 1e-5 identity skip sees the same products.
+    // so the 1e-5 identity skip sees the same products; two runs' products on
+    // one qubit are multiplied only when they are applied.  (A QFT on a
+    // product state is then one layer: the H on a qubit follows its U3 with
+    // only phases on other qubits between them.  30 qubits, complex128: six
+    // sweeps and 39.2 ms with a flush at each such pair, three and 16.1 ms
+    // without.)
     const bool stream = policy_ == POLICY_FUSED;
     // expansions applied at once (u3_expand_group_apply)
     constexpr size_t kGroupMax = 4;
@@ -783,11 +808,13 @@ int Sim::execute()
     // accumulator restarts from the identity once it has come within 1e-5 of it
     auto absorb = [&](size_t q, const std::complex<double> (&u)[4], uint64_t sel, uint64_t delta) {
         Acc &a = pend[q];
-        const bool was = a.active;
-        if (!was)
+        const bool was = a.present();
+        if (a.active && owner[q] != run)
+            a.hold();
+        if (!a.active)
         {
-            a = Acc();
-            a.active = true;
+            a.u00 = a.u11 = 1.0;
+            a.u01 = a.u10 = 0.0;
             a.fixed = true;
             a.sel = sel;
             a.delta = delta;
@@ -799,9 +826,9 @@ int Sim::execute()
         a.u11 = u[2] * o01 + u[3] * o11;
         a.active = !(close_val(a.u00, {1.0, 0.0}) && close_val(a.u01, {0.0, 0.0}) && close_val(a.u10, {0.0, 0.0}) &&
                      close_val(a.u11, {1.0, 0.0}));
-        if (!was && a.active)
+        if (!was && a.present())
             pend_count++;
-        else if (was && !a.active)
+        else if (was && !a.present())
             pend_count--;
         owner[q] = run;
     };
@@ -812,7 +839,7 @@ int Sim::execute()
     };
     auto diag_joins_pre = [&](const DiagGate &d) {
         for (size_t k = 0; k < N_; k++)
-            if (pend[k].active && !diag_commutes(d, pend[k].delta))
+            if (pend[k].present() && !diag_commutes(d, pend[k].delta))
                 return false;
         return true;
     };
@@ -839,8 +866,13 @@ int Sim::execute()
             if (pend[k].active && owner[k] == run)
             {
                 keep.push_back({k, pend[k]});
-                pend[k] = Acc();
-                pend_count--;
+                keep.back().second.held = false;
+                pend[k].active = false; // what is held is of earlier runs
+                if (!pend[k].held)
+                {
+                    pend[k] = Acc();
+                    pend_count--;
+                }
             }
         ZXA_TRY(flush_diag(pre));
         ZXA_TRY(flush_u3(pend, pend_count));
@@ -940,11 +972,13 @@ int Sim::execute()
             if (stream)
             {
                 const uint64_t alpha = sel & amask;
-                bool ok = !(pend[g.q].active && owner[g.q] != run);
+                // another run's product on this qubit: only under the same
+                // descriptor (what is held has that of the product after it)
+                bool ok = !pend[g.q].present() || (pend[g.q].sel == sel && pend[g.q].delta == delta);
                 for (const DiagGate &d : post)
                     ok = ok && diag_commutes(d, delta);
                 for (size_t k = 0; k < N_ && ok; k++)
-                    if (pend[k].active && owner[k] != run)
+                    if (k != g.q && pend[k].present() && (owner[k] != run || pend[k].held))
                         ok = !par(alpha & pend[k].delta) && !par(pend[k].sel & amask & delta);
                 if (!ok)
                     ZXA_TRY(flush_earlier());

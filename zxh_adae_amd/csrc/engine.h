@@ -118,6 +118,24 @@ class Sim
         // place in the circuit (else it is taken from the map at the flush)
         bool fixed = false;
         uint64_t sel = 0, delta = 0;
+        // the products of earlier runs under the same descriptor, each past
+        // its own identity test; applied before u
+        bool held = false;
+        std::complex<double> h00, h01, h10, h11;
+        bool present() const
+        {
+            return active || held;
+        }
+        // u . h as the product of one member
+        void merge();
+        // u becomes (part of) h; the next run's product starts anew
+        void hold()
+        {
+            merge();
+            h00 = u00, h01 = u01, h10 = u10, h11 = u11;
+            held = true;
+            active = false;
+        }
     };
 
     bool solve(size_t q, uint64_t *x) const;
