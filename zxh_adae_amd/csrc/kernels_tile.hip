@@ -75,7 +75,7 @@ struct TGate
 {
     double u[8];    // m00 m01 m10 m11 as (re, im)
     float uf[8];    // the same in float for complex64 states
-    uint64_t amask; // selector bits besides the target, unit-address space
+    uint64_t amask; // selector bits besides the target, unit-address space (kCross: a0)
     uint32_t a0;    // complex64: selector bit 0 (differs between a unit's two amplitudes)
     uint32_t beta;
     uint32_t rpar;  // bit r: parity of amask over register r's offset in the gate's layout
@@ -95,6 +95,17 @@ struct TFan
 };
 constexpr int kFanStride = 2 * (kUnitBits + 1); // doubles of per-tile factors per tile
 
+// Complex64 pair offsets that reach outside the unit and flip its in-unit bit
+// as well (address bit 0 with others, after CX transport): the offset's unit
+// part with this bit set.  The kernel then works in tile coordinates: it
+// exchanges the two amplitudes of every unit whose offset within the tile has
+// the bit (on load and again before the epilogue), so that gates pair first
+// amplitudes with first ones; a selector that sees address bit 0 has the bit
+// in its mask, which makes its parity over an offset the amplitude address's.
+// (Such gates used to take a pair sweep each: 0.85 ms on a 27-qubit state,
+// three of them in a layer's 2.6 ms.)
+constexpr uint64_t kCross = uint64_t(1) << 63;
+
 // Kernel arguments of a pass.  Unit bits 0..seg-1 are unit-address bits
 // 0..seg-1 (seg = 3..6, the tile geometry); the host assigns the others
 // freely (targets first into the register bits of layout 0, then of layout
@@ -104,8 +115,9 @@ struct TPass
 {
     uint32_t ub[kUnitBits];     // unit-address bit of each unit bit (its pivot)
     uint32_t sorted[kUnitBits]; // the same, ascending
-    uint64_t vec[kUnitBits];    // unit-address offset of each unit bit
+    uint64_t vec[kUnitBits];    // unit-address offset of each unit bit (bit 63: see kCross)
     uint64_t ntiles;
+    uint32_t rcross; // bit r: layout-0 register r's offset has kCross
     uint64_t tmask; // unit-address mask of the 12 pivots
     uint64_t gstep; // the grid size deposited into the non-tile bits
     const double *fphase; // fan passes: per-tile factors, kFanStride doubles per tile
@@ -614,6 +626,23 @@ __device__ __forceinline__ void store_tile(const typename UnitT<kC64>::T (&v)[kR
         __builtin_nontemporal_store(v[r], p + (at ^ G->roff[r]));
 }
 
+// Exchanges the amplitudes of the units whose offset has kCross (see there).
+template <bool kC64>
+__device__ __forceinline__ void cross_units(typename UnitT<kC64>::T (&v)[kRegs], uint64_t toff, uint32_t rcross)
+{
+    if constexpr (kC64)
+    {
+        const bool tc = (toff >> 63) != 0;
+#pragma unroll
+        for (int r = 0; r < kRegs; r++)
+        {
+            const bool x = tc != (((rcross >> r) & 1u) != 0);
+            const fvec4 u = v[r];
+            v[r] = fvec4{x ? u.z : u.x, x ? u.w : u.y, x ? u.x : u.z, x ? u.y : u.w};
+        }
+    }
+}
+
 // y of a unit address (see TWin).
 __device__ __forceinline__ uint32_t win_y(ZXA_CONST TWin &W, uint64_t u)
 {
@@ -688,6 +717,8 @@ __device__ __forceinline__ void tile_work(typename UnitT<kC64>::T (&v)[kRegs], t
     ZXA_CONST double *fp = nullptr;
     if constexpr (kFan)
         fp = (ZXA_CONST double *)(P.fphase + tile * kFanStride);
+    if constexpr (kFlip)
+        cross_units<kC64>(v, toff, P.rcross);
     apply_layout<kC64, kFlip, 0, kFan>(v, P, G, base, toff, t, fp, fl);
     if constexpr (kL1)
     {
@@ -710,6 +741,8 @@ __device__ __forceinline__ void tile_work(typename UnitT<kC64>::T (&v)[kRegs], t
         apply_layout<kC64, kFlip, 2, kFan>(v, P, G, base, thr_off<2>(t, P), t, fp, fl);
         transpose<kC64, 2, 0>(v, lds, t);
     }
+    if constexpr (kFlip)
+        cross_units<kC64>(v, toff, P.rcross);
     if constexpr (kDiag)
         epi.apply(v, (ZXA_CONST double *)(tphase + tile * Epi<kC64>::kStride), t);
     if constexpr (kTab)
@@ -747,6 +780,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     const int t = threadIdx.x;
     T *p = static_cast<T *>(state);
     const uint64_t toff = thr_off<0>(t, P);
+    const uint64_t ta = kC64 && kFlip ? toff & ~kCross : toff;
     Epi<kC64> epi;
     if constexpr (kDiag)
         epi.init(ttab, t);
@@ -770,32 +804,32 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     uint64_t t0 = blockIdx.x;
     uint64_t b0 = deposit(t0, P.sorted);
     ZXA_CONST TTab *G = tables(tabp);
-    load_tile<kC64>(a, p, b0 ^ toff, G);
+    load_tile<kC64>(a, p, b0 ^ ta, G);
     uint64_t t1 = t0 + grid;
     bool m1 = t1 < P.ntiles;
     uint64_t b1 = next_base(b0, P);
-    load_tile<kC64>(b, p, (m1 ? b1 : b0) ^ toff, G);
+    load_tile<kC64>(b, p, (m1 ? b1 : b0) ^ ta, G);
     tile_work<kC64, kL1, kL2, kDiag, kFlip, kFan, kTab>(a, lds, P, G, tphase, epi, t, toff, t0, b0, fl, wt, yt);
     for (;;)
     {
         G = tables(tabp);
-        store_tile<kC64>(a, p, b0 ^ toff, G);
+        store_tile<kC64>(a, p, b0 ^ ta, G);
         if (!m1)
             break;
         const uint64_t t2 = t1 + grid;
         const bool m2 = t2 < P.ntiles;
         const uint64_t b2 = next_base(b1, P);
-        load_tile<kC64>(a, p, (m2 ? b2 : b1) ^ toff, G);
+        load_tile<kC64>(a, p, (m2 ? b2 : b1) ^ ta, G);
         tile_work<kC64, kL1, kL2, kDiag, kFlip, kFan, kTab>(b, lds, P, G, tphase, epi, t, toff, t1, b1, fl, wt, yt);
 
         G = tables(tabp);
-        store_tile<kC64>(b, p, b1 ^ toff, G);
+        store_tile<kC64>(b, p, b1 ^ ta, G);
         if (!m2)
             break;
         const uint64_t t3 = t2 + grid;
         const bool m3 = t3 < P.ntiles;
         const uint64_t b3 = next_base(b2, P);
-        load_tile<kC64>(b, p, (m3 ? b3 : b2) ^ toff, G);
+        load_tile<kC64>(b, p, (m3 ? b3 : b2) ^ ta, G);
         tile_work<kC64, kL1, kL2, kDiag, kFlip, kFan, kTab>(a, lds, P, G, tphase, epi, t, toff, t2, b2, fl, wt, yt);
 
         t0 = t2;
@@ -952,12 +986,14 @@ __global__ __launch_bounds__(kThreads) void upper_kernel(void *__restrict__ stat
     const uint64_t tile = blockIdx.x;
     const uint64_t base = deposit(tile, P.sorted);
     const uint64_t toff = thr_off<0>(tl, P);
-    const uint64_t at = base ^ toff;
+    const uint64_t at = base ^ (kC64 && kFlip ? toff & ~kCross : toff);
     ZXA_CONST TTab *G = (ZXA_CONST TTab *)tabp;
     T v[kRegs];
     load_tile<kC64>(v, p, at, G);
     if constexpr (kTab)
         win_load<kC64>(wt, ttab, G->win, threadIdx.x); // synchronized before its use below
+    if constexpr (kFlip)
+        cross_units<kC64>(v, toff, P.rcross);
     // VALU arithmetic here: with the matrix cores the compiler moves the
     // results through AGPRs and the occupancy this kernel relies on halves
     apply_layout<kC64, kFlip, 0, false, false>(v, P, G, base, toff);
@@ -983,6 +1019,8 @@ __global__ __launch_bounds__(kThreads) void upper_kernel(void *__restrict__ stat
 #pragma unroll
     for (int r = 0; r < kRegs; r += 2)
         lane_swap<false>(v[r], v[r + 1]);
+    if constexpr (kFlip)
+        cross_units<kC64>(v, toff, P.rcross);
     if constexpr (kDiag)
     {
         Epi<kC64> epi;
@@ -2457,6 +2495,28 @@ int setup_epilogue(Ctx &ctx, int prec, unsigned n, const std::vector<unsigned> &
     return OK;
 }
 
+// An offset or selector form over amplitude addresses in unit addresses
+// (complex64: address bit 0 becomes kCross).
+uint64_t unit_form(bool c64, uint64_t x)
+{
+    return c64 ? (x >> 1) | ((x & 1u) ? kCross : 0) : x;
+}
+
+// Layout-0 register offsets (unit addresses) from the unit bits' offsets.
+void register_offsets(TPass &P, TTab &G)
+{
+    P.rcross = 0;
+    for (int r = 0; r < kRegs; r++)
+    {
+        uint64_t off = 0;
+        for (int i = 0; i < 4; i++)
+            if ((r >> i) & 1)
+                off ^= P.vec[reg_bit(0, i)];
+        G.roff[r] = off & ~kCross;
+        P.rcross |= uint32_t(off >> 63) << r;
+    }
+}
+
 // Kernel arguments and tables of a pass from its plan (targets' matrices in
 // gs order; every other slot the identity).  use[L]: layout L has a target.
 void fill_pass(int prec, unsigned n, const Plan &pl, TPass &P, TTab &G, bool use[3])
@@ -2470,14 +2530,11 @@ void fill_pass(int prec, unsigned n, const Plan &pl, TPass &P, TTab &G, bool use
     {
         P.ub[k] = pos[k + shift] - shift;
         P.sorted[k] = P.ub[k];
-        P.vec[k] = pl.evec[k + shift] >> shift;
+        P.vec[k] = unit_form(c64, pl.evec[k + shift]);
         P.tmask |= uint64_t(1) << P.ub[k];
     }
     std::sort(P.sorted, P.sorted + kUnitBits);
-    for (int r = 0; r < kRegs; r++)
-        for (int i = 0; i < 4; i++)
-            if ((r >> i) & 1)
-                G.roff[r] ^= P.vec[reg_bit(0, i)];
+    register_offsets(P, G);
     P.ntiles = uint64_t(1) << (n - shift - kUnitBits);
     for (TGate &tg : G.g)
     {
@@ -2851,19 +2908,13 @@ int run_tile_pass(Ctx &ctx, void *state, int prec, unsigned n, const std::vector
             {
                 if (pl.slot[gi] == kIntra)
                     continue;
-                const uint64_t au = (gs[gi].g->packed_sel & ((uint64_t(1) << 63) - 1)) >> shift;
+                const uint64_t au = unit_form(c64, gs[gi].g->packed_sel & ((uint64_t(1) << 63) - 1));
                 if (__builtin_popcountll(au & v0) & 1)
-                    v ^= gs[gi].g->delta >> shift;
+                    v ^= unit_form(c64, gs[gi].g->delta);
             }
             P.vec[k] = v;
         }
-        for (int r = 0; r < kRegs; r++)
-        {
-            G.roff[r] = 0;
-            for (int i = 0; i < 4; i++)
-                if ((r >> i) & 1)
-                    G.roff[r] ^= P.vec[reg_bit(0, i)];
-        }
+        register_offsets(P, G);
     }
     for (size_t gi = 0; gi < gs.size(); gi++)
     {
@@ -2892,7 +2943,7 @@ int run_tile_pass(Ctx &ctx, void *state, int prec, unsigned n, const std::vector
             tg.u[i] = m[i];
             tg.uf[i] = float(m[i]);
         }
-        tg.amask = rest >> shift;
+        tg.amask = unit_form(c64, rest);
         tg.a0 = c64 ? uint32_t(rest & 1u) : 0u;
         tg.beta = beta;
         const int lay = slot == kIntra ? 0 : layout_of_unit_bit(slot);
@@ -3588,8 +3639,10 @@ bool independent_batch(const U3Gate *gates, size_t ngates)
 // takes every remaining gate whose pivot fits: the pivots above the tile's
 // low bits within its upper slots, and no offset reaching above the low bits
 // on a pivot below the first whole 128-byte line of the contiguous run (its
-// lanes would read partial lines of two places).  A pass's first gate
-// always fits, so every pass takes at least one.
+// lanes would read partial lines of two places).  In complex64 only the
+// offset of address bit 0 alone may have it as its pivot (the in-unit slot).  A
+// pass's first gate always fits (its pivot is its own top bit), so every pass
+// takes at least one.
 bool plan_passes(int prec, int geometry, std::vector<const U3Gate *> rest,
                  std::vector<std::vector<SingleGate>> &passes)
 {
@@ -3607,7 +3660,8 @@ bool plan_passes(int prec, int geometry, std::vector<const U3Gate *> rest,
         {
             pass.push_back(g);
             const bool fits = pivot_bits(pass, low, piv, &nhigh) && nhigh <= slots &&
-                              !(piv.back() < std::min(low, whole) && (g->delta >> low) != 0);
+                              !(piv.back() < std::min(low, whole) && (g->delta >> low) != 0) &&
+                              !(c64 && piv.back() == 0 && g->delta != 1);
             if (!fits)
             {
                 pass.pop_back();
@@ -3645,6 +3699,9 @@ bool window_table_host(unsigned n, const DiagGate *gates, size_t ngates, uint64_
     return true;
 }
 
+// Narrowest complex64 state whose kCross offsets ride tile passes.
+constexpr unsigned kCrossBits = 20;
+
 int u3_apply(Ctx &ctx, void *state, int prec, unsigned n, const U3Gate *gates, size_t ngates, const DiagGate *win,
              size_t nwin)
 {
@@ -3666,8 +3723,10 @@ int u3_apply(Ctx &ctx, void *state, int prec, unsigned n, const U3Gate *gates, s
         const U3Gate &g = gates[i];
         const uint64_t alpha = g.packed_sel & ((uint64_t(1) << 63) - 1);
         const bool in_state = g.delta != 0 && (g.delta >> n) == 0 && (alpha >> n) == 0;
-        // complex64 units hold address bit 0: an offset may use it only alone
-        const bool in_units = !c64 || (g.delta & 1u) == 0 || g.delta == 1;
+        // complex64 units hold address bit 0: an offset that has it with
+        // others (kCross) rides a tile pass where a sweep of its own costs
+        // more than the in-unit exchange of the pass (%CROSS%)
+        const bool in_units = !c64 || (g.delta & 1u) == 0 || g.delta == 1 || n >= kCrossBits;
         if (n >= tile_min_bits(prec) && n <= 40 && in_state && in_units)
             ((g.delta & (g.delta - 1)) == 0 ? single : wide).push_back(&g);
         else
