@@ -131,26 +131,38 @@ void ParamRing::release()
     if (host_)
         (void)hipHostFree(host_);
     dev_ = host_ = hdev_ = nullptr;
-    open_.clear();
+    left_.clear();
+    cur_ = 0;
+    off_ = 0;
     end_batch();
 }
 
-// The next slot, once its last consumer has finished; open until done().
-int ParamRing::open_slot(int *slot)
+// Moves on to the next slot once its last consumers have finished.
+int ParamRing::next_slot()
 {
-    const int s = next_;
-    for (int o : open_)
+    const int s = (cur_ + 1) % kSlots;
+    for (int o : left_)
         if (o == s)
         {
             set_error("parameter ring exhausted before done()");
             return EINVAL_;
         }
-    next_ = (next_ + 1) % kSlots;
     if (used_[s])
+    {
         ZXA_HIP(hipEventSynchronize(ev_[s]));
-    open_.push_back(s);
-    *slot = s;
+        used_[s] = false;
+    }
+    left_.push_back(cur_);
+    cur_ = s;
+    off_ = 0;
     return OK;
+}
+
+// Copies bytes [from, to) of the current slot.
+int ParamRing::copy(hipStream_t stream, size_t from, size_t to)
+{
+    const size_t at = size_t(cur_) * kSlotBytes + from;
+    return ring_copy(stream, static_cast<char *>(dev_) + at, static_cast<char *>(hdev_) + at, to - from);
 }
 
 int ParamRing::stage(const void *src, size_t bytes, hipStream_t stream, void **dev)
@@ -160,65 +172,50 @@ int ParamRing::stage(const void *src, size_t bytes, hipStream_t stream, void **d
         set_error("parameter block exceeds ring slot size");
         return EINVAL_;
     }
-    if (batch_ >= 0)
+    if (off_ + bytes > kSlotBytes)
     {
-        size_t off = (boff_ + 255) & ~size_t(255);
-        if (off + bytes > kSlotBytes)
-        {
-            ZXA_TRY(flush(stream));
-            ZXA_TRY(begin_batch());
-            off = 0;
-        }
-        const size_t at = size_t(batch_) * kSlotBytes + off;
-        std::memcpy(static_cast<char *>(host_) + at, src, bytes);
-        boff_ = off + bytes;
-        *dev = static_cast<char *>(dev_) + at;
-        return OK;
+        if (batch_)
+            ZXA_TRY(copy(stream, from_, off_));
+        ZXA_TRY(next_slot());
+        from_ = 0;
     }
-    int s = 0;
-    ZXA_TRY(open_slot(&s));
-    char *h = static_cast<char *>(host_) + size_t(s) * kSlotBytes;
-    char *d = static_cast<char *>(dev_) + size_t(s) * kSlotBytes;
-    std::memcpy(h, src, bytes);
-    ZXA_TRY(ring_copy(stream, d, static_cast<char *>(hdev_) + size_t(s) * kSlotBytes, bytes));
-    *dev = d;
-    return OK;
+    const size_t at = off_;
+    std::memcpy(static_cast<char *>(host_) + size_t(cur_) * kSlotBytes + at, src, bytes);
+    *dev = static_cast<char *>(dev_) + size_t(cur_) * kSlotBytes + at;
+    off_ = std::min(kSlotBytes, (at + bytes + 255) & ~size_t(255));
+    if (batch_)
+        return OK;
+    return copy(stream, at, at + bytes);
 }
 
 int ParamRing::begin_batch()
 {
-    end_batch();
-    int s = 0;
-    ZXA_TRY(open_slot(&s));
-    batch_ = s;
+    batch_ = true;
+    from_ = off_;
     return OK;
 }
 
 int ParamRing::flush(hipStream_t stream)
 {
-    const int s = batch_;
-    const size_t bytes = boff_;
+    const bool open = batch_;
     end_batch();
-    if (s < 0 || bytes == 0)
-        return OK;
-    const size_t at = size_t(s) * kSlotBytes;
-    return ring_copy(stream, static_cast<char *>(dev_) + at, static_cast<char *>(hdev_) + at, bytes);
+    return open ? copy(stream, from_, off_) : OK;
 }
 
 void ParamRing::end_batch()
 {
-    batch_ = -1;
-    boff_ = 0;
+    batch_ = false;
 }
 
+// Every launch that reads the slots left behind has been made: their events.
 int ParamRing::done(hipStream_t stream)
 {
-    for (int s : open_)
+    for (int s : left_)
     {
         ZXA_HIP(hipEventRecord(ev_[s], stream));
         used_[s] = true;
     }
-    open_.clear();
+    left_.clear();
     return OK;
 }
 

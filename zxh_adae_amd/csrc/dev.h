@@ -119,8 +119,11 @@ struct FamilyTiming
     uint64_t bytes = 0; // algorithmic HBM bytes of the timed launches
 };
 
-// Ring of parameter slots: mapped host staging + device copy + event.  A slot
-// is reused only after the event recorded behind its last consumer fired.
+// Ring of parameter slots: mapped host staging + device copy + event.  Blocks
+// are packed into the current slot; one that no longer fits moves on to the
+// next, and the slot left behind gets its event at the next done().  A slot is
+// entered again only after that event fired.  (An event behind every launch
+// kept the next one from starting for 5.7 us.)
 class ParamRing
 {
   public:
@@ -128,31 +131,32 @@ class ParamRing
     static constexpr size_t kSlotBytes = 256 * 1024;
     int init();
     void release();
-    // Copies bytes from src into the next slot (ring_copy on stream) and
-    // returns the device address.  Call done() after the consuming launches.
+    // Copies bytes from src into the ring (ring_copy on stream) and returns
+    // the device address.  Call done() after the consuming launches.
     int stage(const void *src, size_t bytes, hipStream_t stream, void **dev);
     int done(hipStream_t stream);
     // Batched staging: between begin_batch() and flush(), stage() packs the
-    // blocks into one slot at 256-byte aligned offsets and issues no copy (a
-    // block that no longer fits copies the packed ones and opens the next
-    // slot); flush() copies the packed bytes with one ring_copy and ends the
-    // batch.  Launches that read a block come after flush().  end_batch()
-    // drops an unflushed batch (error returns).
+    // blocks and issues no copy (a block that no longer fits copies the packed
+    // ones and goes on in the next slot); flush() copies the packed bytes with
+    // one ring_copy and ends the batch.  Launches that read a block come after
+    // flush().  end_batch() drops an unflushed batch (error returns).
     int begin_batch();
     int flush(hipStream_t stream);
     void end_batch();
 
   private:
-    int open_slot(int *slot);
+    int next_slot();
+    int copy(hipStream_t stream, size_t from, size_t to);
     void *host_ = nullptr;
     void *hdev_ = nullptr; // host_ as the device addresses it (mapped, coherent)
     void *dev_ = nullptr;
     hipEvent_t ev_[kSlots] = {};
     bool used_[kSlots] = {};
-    int next_ = 0;
-    std::vector<int> open_; // staged since the last done()
-    int batch_ = -1;        // slot being packed, or -1
-    size_t boff_ = 0;       // bytes packed in it
+    int cur_ = 0;           // the slot being packed
+    size_t off_ = 0;        // bytes taken in it (a multiple of 256)
+    std::vector<int> left_; // slots left since the last done()
+    bool batch_ = false;
+    size_t from_ = 0; // first byte of the slot not copied yet (batch)
 };
 
 // Copies a staged block from the ring's mapped host slot (src: its device
