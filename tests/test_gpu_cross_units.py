@@ -68,3 +68,20 @@ def test_circuits(gpu_engine, upper, n, kind):
     s.gates(gates)
     s.execute()
     assert np.max(np.abs(s.get_state_array() - o.get_state())) < 2e-5
+
+
+@pytest.mark.parametrize("sel,delta", [(2, 3), (1, 3), (1 << 19, (1 << 19) | 1)])
+def test_a_gate_by_itself_takes_a_sweep(gpu_engine, sel, delta):
+    from zxh_adae_amd import kernels as K
+    rng = np.random.default_rng(sel)
+    psi = rand_state(rng, 20)
+    descs = [(sel, delta, rand_u(rng))]
+    d = dev(gpu_engine, psi.astype(np.complex64), "c64")
+    K.set_timing(True)
+    K.reset_timing()
+    try:
+        d.u3_batch(descs)
+        assert K.timing("u3_pair")["launches"] == 1
+    finally:
+        K.set_timing(False)
+    assert np.max(np.abs(d.download().astype(np.complex128) - oracle_u3(psi, 20, descs))) < TOL64

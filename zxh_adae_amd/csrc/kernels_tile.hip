@@ -3699,7 +3699,9 @@ bool window_table_host(unsigned n, const DiagGate *gates, size_t ngates, uint64_
     return true;
 }
 
-// Narrowest complex64 state whose kCross offsets ride tile passes.
+// Narrowest complex64 state whose kCross offsets ride tile passes (below, a
+// sweep is a launch of 7 us and a batch's two passes of one tile per compute
+// unit are no faster).
 constexpr unsigned kCrossBits = 20;
 
 int u3_apply(Ctx &ctx, void *state, int prec, unsigned n, const U3Gate *gates, size_t ngates, const DiagGate *win,
@@ -3724,9 +3726,12 @@ int u3_apply(Ctx &ctx, void *state, int prec, unsigned n, const U3Gate *gates, s
         const uint64_t alpha = g.packed_sel & ((uint64_t(1) << 63) - 1);
         const bool in_state = g.delta != 0 && (g.delta >> n) == 0 && (alpha >> n) == 0;
         // complex64 units hold address bit 0: an offset that has it with
-        // others (kCross) rides a tile pass where a sweep of its own costs
-        // more than the in-unit exchange of the pass (%CROSS%)
-        const bool in_units = !c64 || (g.delta & 1u) == 0 || g.delta == 1 || n >= kCrossBits;
+        // others (kCross) rides a tile pass beside other gates, where a
+        // batch of n / 2 such gates took 87 us in sweeps of their own and 59
+        // in passes at 20 bits, 219 and 64 at 22, 3221 and 467 at 26.  A gate
+        // by itself is cheaper as a sweep: 18 and 37 us at 20 bits, 210 and
+        // 255 at 26 (a pass's first load and last store are its whole tile).
+        const bool in_units = !c64 || (g.delta & 1u) == 0 || g.delta == 1 || (n >= kCrossBits && ngates > 1);
         if (n >= tile_min_bits(prec) && n <= 40 && in_state && in_units)
             ((g.delta & (g.delta - 1)) == 0 ? single : wide).push_back(&g);
         else
