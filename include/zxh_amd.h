@@ -377,6 +377,9 @@ int zxh_batch_set_info(zxh_batch *b, size_t set, unsigned *nbits, size_t *passes
  *       unit bits 6..11 runs on the LDS-free upper kernel when its highest
  *       target unit-address bit is at least this (0..64, 64 = never;
  *       default 18); results are bit-identical either way
+ *   "circuit.bits.c128" (0..22, default 20), "circuit.bits.c64" (0..23, default
+ *       21): widest state, in address bits, whose circuits execute out of LDS
+ *       where they have more than a layer or so; 0 = never
  *   "block.variant.c128", "block.variant.c64": dense-block kernel variant,
  *       bit 0 prefetch the next wave tile, bit 1 matrix re-read from LDS,
  *       bit 2 cached (not nontemporal) loads and stores (0..7)

@@ -15,10 +15,12 @@ pytestmark = pytest.mark.gpu
 @pytest.fixture(params=[0, 18, 64], ids=lambda u: f"upper{u}")
 def upper(request, gpu_engine):
     from zxh_adae_amd import autotune as A
-    old = A.tune_get("tile.upper.c64")
+    old = {k: A.tune_get(k) for k in ("tile.upper.c64", "circuit.bits.c64")}
     A.tune_set("tile.upper.c64", request.param)
+    A.tune_set("circuit.bits.c64", 0)
     yield
-    A.tune_set("tile.upper.c64", old)
+    for k, v in old.items():
+        A.tune_set(k, v)
 
 
 @pytest.mark.parametrize("n,cx,seed", [(20, 5, 1), (20, 60, 2), (21, 200, 3), (22, 12, 4)])

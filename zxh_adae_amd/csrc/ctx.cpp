@@ -361,6 +361,8 @@ Knob g_knobs[] = {
     {"tile.wide.c64", 1, 0, 1},
     {"tile.upper.c128", 18, 0, 64},
     {"tile.upper.c64", 18, 0, 64},
+    {"circuit.bits.c128", 20, 0, 22},
+    {"circuit.bits.c64", 21, 0, 23},
     {"block.variant.c128", 4, 0, 7},
     {"block.variant.c64", 7, 0, 7},
     {"block.tiles.c128", 0, 0, 4096},

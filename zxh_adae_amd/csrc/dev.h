@@ -230,6 +230,8 @@ struct Ctx
 //                                  whose highest target unit-address bit is at
 //                                  least this runs on the LDS-free upper kernel
 //                                  (64: never)
+//   circuit.bits.c128 / .c64       widest state (address bits) whose circuits
+//                                  execute out of LDS (Sim::suits_lds; 0: none)
 //   block.variant.c128 / .c64      dense-block kernel variant (bit 0 prefetch,
 //                                  bit 1 matrix from LDS, bit 2 cached access)
 //   block.tiles.c128 / .c64        wave tiles per wave of a block sweep (0 =

@@ -221,7 +221,21 @@ int Sim::add_gate(int code, size_t cq, size_t q, double theta, double lambda, do
 
 bool Sim::solve(size_t q, uint64_t *x) const
 {
-    return gf2_solve(rows_, m_, q, x);
+    // the solution is the map's: kept until the map changes (map_changed)
+    if (solved_.size() == N_ && solved_[q])
+    {
+        *x = deltas_[q];
+        return true;
+    }
+    const bool ok = gf2_solve(rows_, m_, q, x);
+    if (ok)
+    {
+        solved_.resize(N_, 0);
+        deltas_.resize(N_, 0);
+        solved_[q] = 1;
+        deltas_[q] = *x;
+    }
+    return ok;
 }
 
 // make_selector + make_local_selector with block_start = 0 (zxh.cpp:55-60, 683-691)
@@ -336,6 +350,7 @@ uint64_t Sim::solve_expand(size_t k, int *rc)
             return 0;
         rows_[k] |= uint64_t(1) << m_;
         m_++;
+        map_changed();
         delta = uint64_t(1) << (m_ - 1);
     }
     return delta;
@@ -345,9 +360,9 @@ int Sim::flush_diag(std::vector<DiagGate> &window)
 {
     if (window.empty())
         return OK;
-    if (use_small_)
+    if (use_lds_)
     {
-        const int src = small_.window(ctx_, dstate_, window.data(), window.size());
+        const int src = circuit_.window(window.data(), window.size());
         window.clear();
         return src;
     }
@@ -531,10 +546,10 @@ bool Sim::take_fan(unsigned t, GateFan &fan)
 // the first (applied after it).
 int Sim::emit_u3(std::vector<U3Gate> &descs)
 {
-    if (use_small_)
+    if (use_lds_)
     {
         for (const U3Gate &g : descs)
-            ZXA_TRY(small_.gate(ctx_, dstate_, g));
+            ZXA_TRY(circuit_.gate(g));
         return OK;
     }
     bool simple = fusable();
@@ -737,6 +752,43 @@ int Sim::flush_u3(std::vector<Acc> &pend, size_t &count)
     return emit_u3(descs);
 }
 
+// Whether the circuit goes to circuit_.  Below the tile passes' narrowest
+// state always (one launch, where each batch and window took its own: 3 to 10
+// times).  Above it where it has more than a layer or so: its tables and plan
+// are paid once, and one layer of a resident state is a pass or two either
+// way (complex128, 20 bits: one layer 60 us in tile passes and 74 here, two
+// 128 and 93, ten 535 and 323; 21 bits 71 and 103, 141 and 151, 600 and 556.
+// complex64, 21 bits: 67 and 85, 129 and 110, 546 and 412; 22 bits 664 and 755
+// for ten).  A state that grows gate by gate costs a launch per new bit
+// besides: one layer of 18 bits 125 and 111, of 20 complex64 122 and 141.
+bool Sim::suits_lds() const
+{
+    if (M_ > size_t(tune_get(prec_ == C64 ? "circuit.bits.c64" : "circuit.bits.c128")))
+        return false;
+    if (M_ < tile_min_bits(prec_) || (!eager_ && M_ <= 18))
+        return true;
+    // gates left when each joins the last one on its qubit if nothing has
+    // touched the qubit since
+    std::vector<uint8_t> touched(N_, 1);
+    size_t left = 0, windows = 0;
+    bool diag = false;
+    for (const GateRec &g : gates_)
+    {
+        const bool pairs = g.type == G_H || g.type == G_U3 || (disable_x_ && (g.type == G_X || g.type == G_CX));
+        left += pairs && touched[g.q] ? 1u : 0u;
+        windows += pairs && diag ? 1u : 0u;
+        diag = pairs ? false : diag || (g.type != G_X && g.type != G_CX);
+        touched[g.q] = !(g.type == G_H || g.type == G_U3);
+        if (g.type == G_CP || g.type == G_CX)
+            touched[g.cq] = 1;
+    }
+    // (at the narrowest a layer is one pass of one tile; a QFT, two gates a
+    // qubit and a window between any two, takes 142 us against 172 at 20 bits
+    // of complex128, where the tile passes form its windows as they go)
+    const bool fans = prec_ != C64 && M_ > 18 && 2 * windows > M_;
+    return 2 * left > (M_ == tile_min_bits(prec_) || fans ? 5 : 3) * M_;
+}
+
 int Sim::execute()
 {
     executed_ = false;
@@ -754,6 +806,7 @@ int Sim::execute()
             rows_[q] = uint64_t(1) << q;
         m_ = N_;
     }
+    map_changed();
 
     pass_u3_.clear();
     pass_fan_.clear();
@@ -763,11 +816,11 @@ int Sim::execute()
     pass_has_fan_ = false;
     exp_group_.clear();
     wide_u3_.clear();
-    use_small_ = policy_ == POLICY_FUSED && M_ <= small_max_bits(prec_);
-    if (use_small_)
+    use_lds_ = policy_ == POLICY_FUSED && suits_lds();
+    if (use_lds_)
     {
         fresh_ = false; // the circuit's first run forms |0...0>
-        small_.begin(unsigned(M_), prec_);
+        circuit_.begin(unsigned(M_), prec_);
     }
 
     // Scheduling.  The reference policy batches each run of consecutive U3
@@ -942,9 +995,9 @@ int Sim::execute()
                     eg.u[2 * i] = u[i].real();
                     eg.u[2 * i + 1] = u[i].imag();
                 }
-                if (use_small_)
+                if (use_lds_)
                 {
-                    ZXA_TRY(small_.gate(ctx_, dstate_, eg));
+                    ZXA_TRY(circuit_.gate(eg));
                     continue;
                 }
                 // the new bit is the top one and its half still zero
@@ -1011,9 +1064,9 @@ int Sim::execute()
                 const uint64_t d = solve_expand(g.q, &rc);
                 if (rc)
                     return rc;
-                if (use_small_)
+                if (use_lds_)
                 {
-                    ZXA_TRY(small_.swap(ctx_, dstate_, d & low_mask(active_bits()), local_selector(g.q), nullptr));
+                    ZXA_TRY(circuit_.swap(d & low_mask(active_bits()), local_selector(g.q), nullptr));
                     break;
                 }
                 ZXA_TRY(flush_group());
@@ -1033,10 +1086,10 @@ int Sim::execute()
                 const uint64_t d = solve_expand(g.q, &rc);
                 if (rc)
                     return rc;
-                if (use_small_)
+                if (use_lds_)
                 {
                     const uint64_t scq = local_selector(g.cq);
-                    ZXA_TRY(small_.swap(ctx_, dstate_, d & low_mask(active_bits()), local_selector(g.q), &scq));
+                    ZXA_TRY(circuit_.swap(d & low_mask(active_bits()), local_selector(g.q), &scq));
                     break;
                 }
                 ZXA_TRY(flush_group());
@@ -1048,6 +1101,7 @@ int Sim::execute()
             {
                 rows_[g.q] ^= rows_[g.cq];
                 b_[g.q] = uint8_t(b_[g.q] != b_[g.cq]);
+                map_changed();
             }
             break;
         case G_CP: {
@@ -1075,8 +1129,8 @@ int Sim::execute()
         }
     }
     ZXA_TRY(flush_all());
-    if (use_small_)
-        ZXA_TRY(small_.run(ctx_, dstate_));
+    if (use_lds_)
+        ZXA_TRY(circuit_.run(ctx_, dstate_));
     ZXA_TRY(flush_pass());
     ZXA_TRY(flush_group());
     ZXA_TRY(settle());

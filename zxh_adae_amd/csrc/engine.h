@@ -10,8 +10,9 @@
 #pragma once
 
 #include "dev.h"
-#include "small.h"
+#include "circuit.h"
 
+#include <algorithm>
 #include <complex>
 #include <cstdint>
 #include <vector>
@@ -168,6 +169,13 @@ class Sim
     std::vector<uint64_t> rows_;
     std::vector<uint8_t> b_;
     size_t m_ = 0;
+    // pair offsets solved since the map last changed
+    mutable std::vector<uint8_t> solved_;
+    mutable std::vector<uint64_t> deltas_;
+    void map_changed()
+    {
+        std::fill(solved_.begin(), solved_.end(), uint8_t(0));
+    }
     // physical state
     void *dstate_ = nullptr;
     bool fresh_ = false;      // the state is |0...0> of fresh_elems_ amplitudes, not yet written
@@ -205,10 +213,11 @@ class Sim
     std::vector<U3Gate> exp_group_;
     unsigned exp_base_ = 0;
     int flush_group();
-    // fused policy, a state that fits one compute unit's LDS: every
-    // operation goes to small_ and runs at the end of execute()
-    bool use_small_ = false;
-    SmallCircuit small_;
+    // fused policy, a small or middling state: every operation goes to
+    // circuit_ and runs at the end of execute()
+    bool use_lds_ = false;
+    bool suits_lds() const;
+    LdsCircuit circuit_;
     Ctx ctx_;
 };
 
