@@ -111,18 +111,18 @@ int Ansatz::build_schedule()
 {
     std::vector<Pass> best, p;
     unsigned bseg = 0;
-    if (force_seg_ >= 3 && force_seg_ <= 6)
+    auto sweeps = [](const std::vector<Pass> &ps) {
+        return size_t(std::count_if(ps.begin(), ps.end(), [](const Pass &q) { return !q.joins; }));
+    };
+    if (force_seg_ != 0)
     {
         schedule_for(force_seg_, best);
-        passes_.swap(best);
-        seg_ = force_seg_;
-        tile_passes_ = passes_.size();
-        return OK;
+        bseg = force_seg_;
     }
-    for (unsigned seg = 6; seg >= 3; seg--)
+    for (unsigned seg = 6; seg >= 3 && force_seg_ == 0; seg--)
     {
         schedule_for(seg, p);
-        if (bseg == 0 || p.size() < best.size())
+        if (bseg == 0 || sweeps(p) < sweeps(best))
         {
             best.swap(p);
             bseg = seg;
@@ -130,7 +130,11 @@ int Ansatz::build_schedule()
     }
     passes_.swap(best);
     seg_ = bseg;
-    tile_passes_ = passes_.size();
+    sweeps_.clear();
+    for (size_t k = 0; k < passes_.size(); k++)
+        if (!passes_[k].joins)
+            sweeps_.push_back(k);
+    tile_passes_ = sweeps_.size();
     return OK;
 }
 
@@ -155,19 +159,54 @@ void Ansatz::schedule_for(unsigned seg, std::vector<Pass> &passes_) const
             }
         if (lows.empty() && highs.empty() && window.empty())
             return;
-        size_t hi = 0;
-        bool first = true;
-        while (first || hi < highs.size())
+        // chunks of the high targets: by fixed ranges of qubits (so that
+        // layers after each other have the same ones) where that takes no
+        // more of them than packing
+        std::vector<std::vector<Target>> chunks, packed;
+        for (size_t k = 0; k < highs.size(); k++)
         {
-            Pass p;
-            if (first)
-                p.targets = lows;
-            const size_t take = std::min<size_t>(slots, highs.size() - hi);
-            for (size_t k = 0; k < take; k++)
-                p.targets.push_back(highs[hi + k]);
-            hi += take;
-            first = false;
-            passes_.push_back(p);
+            if (k == 0 || (highs[k].q - low) / slots != (highs[k - 1].q - low) / slots)
+                chunks.emplace_back();
+            chunks.back().push_back(highs[k]);
+            if (k % slots == 0)
+                packed.emplace_back();
+            packed.back().push_back(highs[k]);
+        }
+        if (packed.size() < chunks.size())
+            chunks.swap(packed);
+        if (chunks.empty())
+            chunks.emplace_back();
+        // the low targets in a pass that begins or ends no layer, if there is one
+        std::vector<Target> &c = chunks[chunks.size() >= 3 ? 1 : 0];
+        c.insert(c.begin(), lows.begin(), lows.end());
+        // The layer before ended with its window, which any tile can apply:
+        // where a chunk's targets and that last pass's share a tile, the
+        // chunk comes first and joins the pass, behind the window, and the
+        // layers run through the chunks back and forth (a layer of k sweeps
+        // then takes k - 1).
+        size_t at = chunks.size();
+        const size_t np = passes_.size();
+        if (chunks.size() >= 2 && np > 0 && !passes_[np - 1].joins && !passes_[np - 1].window.empty() &&
+            (np < 2 || passes_[np - 2].window.empty()))
+            for (size_t k = chunks.size(); k-- > 0;)
+            {
+                uint64_t used = 0;
+                for (const std::vector<Target> *ts : {&passes_[np - 1].targets, &chunks[k]})
+                    for (const Target &t : *ts)
+                        used |= uint64_t(t.q >= low) << t.q;
+                if (at == chunks.size() && unsigned(__builtin_popcountll(used)) <= slots)
+                    at = k;
+            }
+        const bool joins = at < chunks.size();
+        if (joins && at == chunks.size() - 1)
+            std::reverse(chunks.begin(), chunks.end());
+        else if (joins)
+            std::rotate(chunks.begin(), chunks.begin() + long(at), chunks.begin() + long(at) + 1);
+        for (size_t k = 0; k < chunks.size(); k++)
+        {
+            passes_.emplace_back();
+            passes_.back().targets = chunks[k];
+            passes_.back().joins = joins && k == 0;
         }
         passes_.back().window = window;
         for (unsigned q = 0; q < n_; q++)
@@ -325,15 +364,31 @@ void Ansatz::pass_adjoint(size_t pi, const double *params, std::vector<AdjTarget
 
 int Ansatz::run_forward(const double *params)
 {
-    ZXA_TRY(state_reset(ctx_, psi_, prec_, size_t(1) << n_));
-    std::vector<U3Gate> gs;
+    std::vector<U3Gate> gs, gs2;
     std::vector<DiagGate> w;
-    for (size_t p = 0; p < passes_.size(); p++)
+    // the first sweep forms |0...0> itself
+    bool fresh = true;
+    for (size_t g = 0; g < sweeps_.size(); g++)
     {
+        bool two;
+        const size_t p = sweep(g, &two);
         pass_gates(p, params, gs);
         pass_window(p, params, false, w);
-        ZXA_TRY(fused_pass_apply(ctx_, psi_, prec_, n_, gs.data(), gs.size(), w.data(), w.size(), int(seg_)));
+        if (two)
+        {
+            if (fresh)
+                ZXA_TRY(state_reset(ctx_, psi_, prec_, size_t(1) << n_));
+            pass_gates(p + 1, params, gs2);
+            ZXA_TRY(turn_pass_apply(ctx_, psi_, prec_, n_, gs.data(), gs.size(), w.data(), w.size(), gs2.data(),
+                                    gs2.size(), int(seg_)));
+        }
+        else
+            ZXA_TRY(fused_pass_apply(ctx_, psi_, prec_, n_, gs.data(), gs.size(), w.data(), w.size(), int(seg_),
+                                     nullptr, fresh));
+        fresh = false;
     }
+    if (fresh)
+        ZXA_TRY(state_reset(ctx_, psi_, prec_, size_t(1) << n_));
     return OK;
 }
 
@@ -360,6 +415,14 @@ int Ansatz::backward(const double *params, double *grads, double *energy)
     state_valid_ = false;
     if (!same)
         ZXA_TRY(run_forward(params));
+    // the circuit's last window is undone before H, a sum of Z products that
+    // commutes with it: lam = H psi then has it undone as well
+    std::vector<DiagGate> w;
+    if (!passes_.empty() && !passes_.back().window.empty())
+    {
+        pass_window(passes_.size() - 1, params, true, w);
+        ZXA_TRY(diag_apply(ctx_, psi_, prec_, n_, w.data(), w.size()));
+    }
     double e2[2] = {0.0, 0.0};
     ZXA_TRY(observable_apply(ctx_, psi_, lam_, prec_, n_, qi_.data(), qj_.data(), coef_.data(), coef_.size(), e2));
     if (energy)
@@ -368,22 +431,28 @@ int Ansatz::backward(const double *params, double *grads, double *energy)
         energy[1] = e2[1];
     }
     ZXA_HIP(hipMemsetAsync(dgrads_, 0, std::max<size_t>(1, nparams_) * sizeof(double), ctx_.stream));
-    std::vector<DiagGate> w;
-    if (!passes_.empty() && !passes_.back().window.empty())
+    std::vector<AdjTarget> ts, ts2;
+    for (size_t g = sweeps_.size(); g-- > 0;)
     {
-        pass_window(passes_.size() - 1, params, true, w);
-        ZXA_TRY(diag_apply(ctx_, psi_, prec_, n_, w.data(), w.size()));
-        ZXA_TRY(diag_apply(ctx_, lam_, prec_, n_, w.data(), w.size()));
-    }
-    std::vector<AdjTarget> ts;
-    for (size_t jj = passes_.size(); jj-- > 0;)
-    {
-        pass_adjoint(jj, params, ts);
+        bool two;
+        const size_t jj = sweep(g, &two);
         w.clear();
-        if (jj > 0)
-            pass_window(jj - 1, params, true, w);
+        ts2.clear();
+        if (two)
+        {
+            // the second round undone, the window, then the first
+            pass_adjoint(jj + 1, params, ts);
+            pass_window(jj, params, true, w);
+            pass_adjoint(jj, params, ts2);
+        }
+        else
+        {
+            pass_adjoint(jj, params, ts);
+            if (jj > 0)
+                pass_window(jj - 1, params, true, w);
+        }
         ZXA_TRY(adjoint_pass_apply(ctx_, psi_, lam_, prec_, n_, ts.data(), ts.size(), w.data(), w.size(), dgrads_,
-                                   nparams_, int(seg_)));
+                                   nparams_, int(seg_), ts2.data(), ts2.size()));
     }
     if (nparams_ > 0)
         ZXA_HIP(hipMemcpyAsync(grads, dgrads_, nparams_ * sizeof(double), hipMemcpyDeviceToHost, ctx_.stream));

@@ -97,6 +97,18 @@ class Ansatz
     {
         return seg_;
     }
+    size_t passes() const
+    {
+        return passes_.size();
+    }
+    // Sweep g of the forward schedule: its first pass, and whether the pass
+    // after it runs in the same sweep, on the same tiles, behind the first
+    // one's window (schedule_for).
+    size_t sweep(size_t g, bool *two) const
+    {
+        *two = sweeps_[g] + 1 < passes_.size() && passes_[sweeps_[g] + 1].joins;
+        return sweeps_[g];
+    }
     // Pass p of the forward schedule: its U3 gates (fused matrices at params)
     // and its diagonal window (angles negated when negate).
     void pass_gates(size_t p, const double *params, std::vector<U3Gate> &gates) const;
@@ -131,6 +143,7 @@ class Ansatz
     {
         std::vector<Target> targets;
         std::vector<size_t> window; // CZ / CP operations
+        bool joins = false;         // second round of the sweep that the pass before begins
     };
     Mat op_matrix(size_t i, const double *params) const;
     int build_schedule();
@@ -143,6 +156,7 @@ class Ansatz
     size_t nparams_;
     std::vector<AnsatzOp> ops_;
     std::vector<Pass> passes_; // tile passes, in forward order
+    std::vector<size_t> sweeps_; // per sweep over the state: its first pass
     size_t tile_passes_ = 0;
     unsigned seg_ = 0;       // tile geometry the schedule was built for
     unsigned force_seg_ = 0; // geometry asked for by set_geometry (0: the rule)

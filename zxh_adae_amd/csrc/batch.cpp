@@ -40,7 +40,6 @@ AnsatzBatch::~AnsatzBatch()
     }
     fwd_.clear();
     bwd_.clear();
-    init_.reset();
     obs_fwd_.reset();
     obs_bwd_.reset();
     for (void *p : {arena_, static_cast<void *>(d_grads_), static_cast<void *>(d_energy_),
@@ -123,92 +122,86 @@ int AnsatzBatch::finalize()
     for (Set &s : sets_)
         maxp = std::max(maxp, s.a->tile_passes());
     std::vector<U3Gate> gs;
-    std::vector<DiagGate> w;
     for (size_t p = 0; p < maxp; p++)
     {
         std::vector<BatchPassSpec> specs;
-        std::vector<std::pair<size_t, size_t>> map;
+        std::vector<Item> map;
         for (size_t i = 0; i < sets_.size(); i++)
         {
             Set &s = sets_[i];
             if (s.a->tile_passes() <= p)
                 continue;
             const std::vector<double> zero(std::max<size_t>(1, s.a->nparams()), 0.0);
-            s.a->pass_gates(p, zero.data(), gs);
-            s.a->pass_window(p, zero.data(), false, w);
+            Item m;
+            m.set = i;
+            m.pass[0] = s.a->sweep(p, &m.two);
+            m.pass[1] = m.pass[0] + 1;
             BatchPassSpec sp;
+            s.a->pass_gates(m.pass[0], zero.data(), gs);
+            sp.targets = targets_of(gs);
+            // (the circuit's last window commutes with the observable, a sum
+            // of Z products: neither energy nor gradient sees it, and the
+            // states stay here)
+            if (m.pass[0] + 1 < s.a->passes())
+                s.a->pass_window(m.pass[0], zero.data(), false, sp.window);
+            if (m.two)
+            {
+                s.a->pass_gates(m.pass[1], zero.data(), gs);
+                sp.targets2 = targets_of(gs);
+            }
             sp.psi = s.psi;
             sp.n = s.a->nbits();
             sp.geometry = int(s.a->geometry());
-            sp.targets = targets_of(gs);
-            sp.window = w;
             specs.push_back(sp);
-            map.push_back({i, p});
+            map.push_back(m);
         }
         fwd_.emplace_back(new BatchLaunch());
         ZXA_TRY(batch_prepare(ctx_, prec_, false, specs, *fwd_.back()));
         fwd_map_.push_back(map);
     }
-    // backward step r runs pass P_s - 1 - r of every set with P_s > r; its
-    // epilogue is the previous pass's window with negated angles
+    // backward step r runs sweep P_s - 1 - r of every set with P_s > r: a
+    // sweep of two rounds undoes the second, the window between them and the
+    // first; the epilogue of the others is the previous pass's window with
+    // negated angles
     for (size_t r = 0; r < maxp; r++)
     {
         std::vector<BatchPassSpec> specs;
-        std::vector<std::pair<size_t, size_t>> map;
+        std::vector<Item> map;
         for (size_t i = 0; i < sets_.size(); i++)
         {
             Set &s = sets_[i];
             const size_t P = s.a->tile_passes();
             if (P <= r)
                 continue;
-            const size_t j = P - 1 - r;
             const std::vector<double> zero(std::max<size_t>(1, s.a->nparams()), 0.0);
-            s.a->pass_gates(j, zero.data(), gs);
+            Item m;
+            m.set = i;
+            const size_t j = s.a->sweep(P - 1 - r, &m.two);
+            m.pass[0] = m.two ? j + 1 : j;
+            m.pass[1] = j;
             BatchPassSpec sp;
+            s.a->pass_gates(m.pass[0], zero.data(), gs);
+            sp.targets = targets_of(gs);
+            if (m.two)
+            {
+                s.a->pass_gates(j, zero.data(), gs);
+                sp.targets2 = targets_of(gs);
+                s.a->pass_window(j, zero.data(), true, sp.window);
+            }
+            else if (j > 0)
+                s.a->pass_window(j - 1, zero.data(), true, sp.window);
             sp.psi = s.psi;
             sp.lam = s.lam;
             sp.n = s.a->nbits();
             sp.geometry = int(s.a->geometry());
-            sp.targets = targets_of(gs);
-            if (j > 0)
-                s.a->pass_window(j - 1, zero.data(), true, sp.window);
             sp.grads = s.grads;
             sp.nparams = s.a->nparams();
             specs.push_back(sp);
-            map.push_back({i, j});
+            map.push_back(m);
         }
         bwd_.emplace_back(new BatchLaunch());
         ZXA_TRY(batch_prepare(ctx_, prec_, true, specs, *bwd_.back()));
         bwd_map_.push_back(map);
-    }
-    // the last pass's window of every set, undone on both states first
-    {
-        std::vector<BatchPassSpec> specs;
-        for (size_t i = 0; i < sets_.size(); i++)
-        {
-            Set &s = sets_[i];
-            const size_t P = s.a->tile_passes();
-            if (P == 0)
-                continue;
-            const std::vector<double> zero(std::max<size_t>(1, s.a->nparams()), 0.0);
-            BatchPassSpec sp;
-            s.a->pass_window(P - 1, zero.data(), true, sp.window);
-            if (sp.window.empty())
-                continue;
-            sp.psi = s.psi;
-            sp.lam = s.lam;
-            sp.n = s.a->nbits();
-            sp.geometry = int(s.a->geometry());
-            sp.grads = s.grads;
-            sp.nparams = s.a->nparams();
-            specs.push_back(sp);
-            init_map_.push_back(i);
-        }
-        if (!specs.empty())
-        {
-            init_.reset(new BatchLaunch());
-            ZXA_TRY(batch_prepare(ctx_, prec_, true, specs, *init_));
-        }
     }
     std::vector<ObsSpec> of, ob;
     for (Set &s : sets_)
@@ -248,8 +241,6 @@ int AnsatzBatch::enqueue(bool backward)
         rc = zero_fill(ctx_, d_grads_, align256(std::max<size_t>(1, total_params_) * 8));
         if (!rc)
             rc = obs_batch_launch(ctx_, *obs_bwd_);
-        if (!rc && init_)
-            rc = batch_launch(ctx_, *init_);
         for (size_t r = 0; r < bwd_.size() && !rc; r++)
             rc = batch_launch(ctx_, *bwd_[r]);
     }
@@ -292,9 +283,13 @@ int AnsatzBatch::fill_tables(const double *params, bool backward)
     {
         for (size_t k = 0; k < fwd_map_[p].size(); k++)
         {
-            const Set &s = sets_[fwd_map_[p][k].first];
-            s.a->pass_gates(fwd_map_[p][k].second, params + s.poff, gs);
-            batch_set_gates(*fwd_[p], k, gs.data(), gs.size());
+            const Item &m = fwd_map_[p][k];
+            const Set &s = sets_[m.set];
+            for (int r = 0; r < (m.two ? 2 : 1); r++)
+            {
+                s.a->pass_gates(m.pass[r], params + s.poff, gs);
+                batch_set_gates(*fwd_[p], k, r, gs.data(), gs.size());
+            }
         }
         ZXA_TRY(batch_upload(ctx_, *fwd_[p]));
     }
@@ -305,14 +300,16 @@ int AnsatzBatch::fill_tables(const double *params, bool backward)
     {
         for (size_t k = 0; k < bwd_map_[r].size(); k++)
         {
-            const Set &s = sets_[bwd_map_[r][k].first];
-            s.a->pass_adjoint(bwd_map_[r][k].second, params + s.poff, ts);
-            ZXA_TRY(batch_set_adjoint(*bwd_[r], k, ts.data(), ts.size()));
+            const Item &m = bwd_map_[r][k];
+            const Set &s = sets_[m.set];
+            for (int j = 0; j < (m.two ? 2 : 1); j++)
+            {
+                s.a->pass_adjoint(m.pass[j], params + s.poff, ts);
+                ZXA_TRY(batch_set_adjoint(*bwd_[r], k, j, ts.data(), ts.size()));
+            }
         }
         ZXA_TRY(batch_upload(ctx_, *bwd_[r]));
     }
-    if (init_)
-        ZXA_TRY(batch_upload(ctx_, *init_));
     return OK;
 }
 

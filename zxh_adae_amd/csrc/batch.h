@@ -54,7 +54,7 @@ class AnsatzBatch
     }
     size_t launches() const
     {
-        return fwd_.size() + bwd_.size() + (init_ ? 1 : 0) + 2;
+        return fwd_.size() + bwd_.size() + 2;
     }
     Ctx &ctx()
     {
@@ -85,11 +85,14 @@ class AnsatzBatch
     double *d_energy_ = nullptr;
     uint64_t *d_states_ = nullptr; // psi pointers, for the reset
     std::vector<std::unique_ptr<BatchLaunch>> fwd_, bwd_;
-    std::unique_ptr<BatchLaunch> init_;
     std::unique_ptr<ObsBatch> obs_fwd_, obs_bwd_;
-    // per launch, per item: (set, pass) it carries
-    std::vector<std::vector<std::pair<size_t, size_t>>> fwd_map_, bwd_map_;
-    std::vector<size_t> init_map_;
+    // per launch, per item: its set and the pass or two passes it carries
+    struct Item
+    {
+        size_t set = 0, pass[2] = {0, 0};
+        bool two = false;
+    };
+    std::vector<std::vector<Item>> fwd_map_, bwd_map_;
     hipGraph_t graph_[2] = {nullptr, nullptr};
     hipGraphExec_t exec_[2] = {nullptr, nullptr};
     Ctx ctx_;

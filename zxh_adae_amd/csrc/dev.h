@@ -337,6 +337,11 @@ struct GateFan
 int fused_pass_apply(Ctx &ctx, void *state, int prec, unsigned nbits, const U3Gate *gates, size_t ngates,
                      const DiagGate *diag, size_t ndiag, int geometry = -1, const GateFan *fans = nullptr,
                      bool fresh = false);
+// Two rounds of single-bit gates (commuting within a round, both rounds'
+// targets within one tile's) with a phase-polynomial window between them, in
+// one sweep.
+int turn_pass_apply(Ctx &ctx, void *state, int prec, unsigned nbits, const U3Gate *gates, size_t ngates,
+                    const DiagGate *diag, size_t ndiag, const U3Gate *gates2, size_t ngates2, int geometry);
 // One target of an adjoint pass: the uncompute matrix m (= U^dagger of the
 // forward pass's fused single-qubit gate on this qubit, (re, im) x 4), up to
 // two transition operators a[k] (2x2 traceless Hermitian; zero when unused)
@@ -353,9 +358,10 @@ struct AdjTarget
 // addressing, single-bit targets): transition values, then m on both states,
 // then the diagonal window (given with the angles to apply) on both.
 // dgrads: device array of parameter gradients, accumulated in stream order.
+// targets2 (of a turn, in the tile of both): a second round after the window.
 int adjoint_pass_apply(Ctx &ctx, void *psi, void *lam, int prec, unsigned nbits, const AdjTarget *targets,
                        size_t ntargets, const DiagGate *diag, size_t ndiag, double *dgrads, size_t nparams,
-                       int geometry = -1);
+                       int geometry = -1, const AdjTarget *targets2 = nullptr, size_t ntargets2 = 0);
 // Dense 5-qubit block: y[t] = sum_t' u[t][t'] x[t'] over every group of 32
 // amplitudes differing in the target bits (bit b of t = targets[b]); u is
 // 32x32 complex, row-major (re, im) pairs.  One sweep, matrix cores.
@@ -372,6 +378,7 @@ struct BatchPassSpec
     unsigned n = 0;
     std::vector<unsigned> targets;
     std::vector<DiagGate> window;
+    std::vector<unsigned> targets2; // a second round, after the window (none: empty)
     double *grads = nullptr; // adjoint: the state's gradient array (device)
     size_t nparams = 0;      // adjoint: its length
     int geometry = -1;       // tile geometry of the state's passes (-1: the knob's)
@@ -380,22 +387,31 @@ struct BatchLaunch
 {
     int prec = 0;
     bool adj = false;
-    bool l1 = false, l2 = false; // some item uses register layout 1 / 2
     size_t nitems = 0;
-    uint64_t total_tiles = 0;
-    int grid = 0;
+    // One kernel launch each: items of one round or two, with or without
+    // targets in register layout 2.
+    struct Part
+    {
+        bool turn = false, l1 = false, l2 = false;
+        size_t first = 0, nitems = 0; // in d_items
+        uint64_t total_tiles = 0;
+        int grid = 0;
+    };
+    static constexpr int kParts = 4;
+    Part parts[kParts];
     void *d_items = nullptr, *d_tabs = nullptr, *d_adjs = nullptr, *d_partial = nullptr, *d_collect = nullptr,
          *d_epi = nullptr;
     void *h_tables = nullptr; // pinned mirror of d_tabs | d_adjs (d_adjs points into d_tabs)
     size_t tab_bytes = 0, adj_bytes = 0;
-    std::vector<std::vector<int>> slots; // per item: slot of each target
+    std::vector<std::vector<int>> slots[2]; // per round and item: slot of each target
+    std::vector<size_t> tab[2];             // per round and item: its table (second round: none below nitems)
     std::vector<size_t> nparams;         // adjoint: per item, length of its gradient array
     ~BatchLaunch();
 };
 int batch_prepare(Ctx &ctx, int prec, bool adj, const std::vector<BatchPassSpec> &specs, BatchLaunch &out);
-// Matrices of item i for this run (into the pinned mirror).
-void batch_set_gates(BatchLaunch &b, size_t item, const U3Gate *gates, size_t ngates);
-int batch_set_adjoint(BatchLaunch &b, size_t item, const AdjTarget *targets, size_t ntargets);
+// Matrices of item i's round (0 or 1) for this run (into the pinned mirror).
+void batch_set_gates(BatchLaunch &b, size_t item, int round, const U3Gate *gates, size_t ngates);
+int batch_set_adjoint(BatchLaunch &b, size_t item, int round, const AdjTarget *targets, size_t ntargets);
 // Copies the mirror to the device tables (async on ctx.stream).
 int batch_upload(Ctx &ctx, BatchLaunch &b);
 // The batched kernel (and, for adjoint launches, the gradient collection).

@@ -706,8 +706,9 @@ __device__ __forceinline__ void win_apply(typename UnitT<kC64>::T (&v)[kRegs], c
 
 // Gates, transposes and the diagonal epilogue of one tile held in v
 // (kDiag: the phase-polynomial epilogue; kTab: the window table wt, with
-// yt the thread offset's y).
-template <bool kC64, bool kL1, bool kL2, bool kDiag, bool kFlip, bool kFan = false, bool kTab = false>
+// yt the thread offset's y).  kTurn: a second round of gates (G[1]) after it.
+template <bool kC64, bool kL1, bool kL2, bool kDiag, bool kFlip, bool kFan = false, bool kTab = false,
+          bool kTurn = false>
 __device__ __forceinline__ void tile_work(typename UnitT<kC64>::T (&v)[kRegs], typename UnitT<kC64>::T *lds,
                                           const TPass &P, ZXA_CONST TTab *G, const double *tphase,
                                           const Epi<kC64> &epi, int t, uint64_t toff, uint64_t tile, uint64_t base,
@@ -747,6 +748,8 @@ __device__ __forceinline__ void tile_work(typename UnitT<kC64>::T (&v)[kRegs], t
         epi.apply(v, (ZXA_CONST double *)(tphase + tile * Epi<kC64>::kStride), t);
     if constexpr (kTab)
         win_apply<kC64>(v, wt, G->win, win_y(G->win, base) ^ yt);
+    if constexpr (kTurn)
+        tile_work<kC64, kL1, kL2, false, kFlip>(v, lds, P, G + 1, tphase, epi, t, toff, tile, base);
 }
 
 // The tables are re-read at every tile (see TTab): the pointer is laundered
@@ -766,7 +769,11 @@ __device__ __forceinline__ ZXA_CONST TTab *tables(const TTab *tabp)
 // that waiting for a tile's loads never waits for the previous stores.  The
 // prefetch is unconditional (past the last tile it re-reads the current one):
 // with no branch around it the compiler's wait counts stay exact.
-template <bool kC64, bool kL1, bool kL2, bool kDiag, bool kFlip, bool kFan = false, bool kTab = false>
+// kTurn (two rounds with a window between them; complex64, 28 qubits, seven or
+// eight gates a round): 1.35 ms, where the two sweeps of one round took 0.93
+// and 0.86, both bound by memory.
+template <bool kC64, bool kL1, bool kL2, bool kDiag, bool kFlip, bool kFan = false, bool kTab = false,
+          bool kTurn = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void tile_kernel(
     void *__restrict__ state, const TPass P, const TTab *__restrict__ tabp, const double *__restrict__ ttab,
     const double *__restrict__ tphase)
@@ -809,7 +816,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     bool m1 = t1 < P.ntiles;
     uint64_t b1 = next_base(b0, P);
     load_tile<kC64>(b, p, (m1 ? b1 : b0) ^ ta, G);
-    tile_work<kC64, kL1, kL2, kDiag, kFlip, kFan, kTab>(a, lds, P, G, tphase, epi, t, toff, t0, b0, fl, wt, yt);
+    tile_work<kC64, kL1, kL2, kDiag, kFlip, kFan, kTab, kTurn>(a, lds, P, G, tphase, epi, t, toff, t0, b0, fl, wt, yt);
     for (;;)
     {
         G = tables(tabp);
@@ -820,7 +827,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         const bool m2 = t2 < P.ntiles;
         const uint64_t b2 = next_base(b1, P);
         load_tile<kC64>(a, p, (m2 ? b2 : b1) ^ ta, G);
-        tile_work<kC64, kL1, kL2, kDiag, kFlip, kFan, kTab>(b, lds, P, G, tphase, epi, t, toff, t1, b1, fl, wt, yt);
+        tile_work<kC64, kL1, kL2, kDiag, kFlip, kFan, kTab, kTurn>(b, lds, P, G, tphase, epi, t, toff, t1, b1, fl, wt, yt);
 
         G = tables(tabp);
         store_tile<kC64>(b, p, b1 ^ ta, G);
@@ -830,7 +837,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         const bool m3 = t3 < P.ntiles;
         const uint64_t b3 = next_base(b2, P);
         load_tile<kC64>(b, p, (m3 ? b3 : b2) ^ ta, G);
-        tile_work<kC64, kL1, kL2, kDiag, kFlip, kFan, kTab>(a, lds, P, G, tphase, epi, t, toff, t2, b2, fl, wt, yt);
+        tile_work<kC64, kL1, kL2, kDiag, kFlip, kFan, kTab, kTurn>(a, lds, P, G, tphase, epi, t, toff, t2, b2, fl, wt, yt);
 
         t0 = t2;
         b0 = b2;
@@ -1575,8 +1582,12 @@ __device__ __forceinline__ void adj_tile(typename UnitT<kC64>::T (&v)[kRegs], ty
     }
 }
 
-// partial: one row of 64 lane accumulators per wave.
-template <bool kC64, bool kL1, bool kL2, bool kDiag>
+// partial: one row of 64 lane accumulators per wave.  kTurn (with kDiag): a
+// second round of gates after the window, its rows behind the first round's
+// (28 qubits of complex64: 3.22 ms, two sweeps 2.0 and 2.28; the vector and
+// matrix units are busy for most of it, and for half of a sweep of one round,
+// whose states' way to memory and back is 1.5 ms).
+template <bool kC64, bool kL1, bool kL2, bool kDiag, bool kTurn = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void adj_kernel(
     void *__restrict__ psi, void *__restrict__ lam, const TPass P, const TTab *__restrict__ tabp,
     const double *__restrict__ ttab, const double *__restrict__ tphase, double *__restrict__ partial)
@@ -1587,7 +1598,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     T *pp = static_cast<T *>(psi);
     T *pl = static_cast<T *>(lam);
     const uint64_t toff = thr_off<0>(t, P);
-    double acc = 0.0;
+    double acc = 0.0, acc2 = 0.0;
     uint64_t base = deposit(uint64_t(blockIdx.x), P.sorted);
     for (uint64_t tile = blockIdx.x; tile < P.ntiles; tile += gridDim.x)
     {
@@ -1606,63 +1617,103 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
             asm volatile("" : "+s"(et));
             Epi<kC64> epi;
             epi.init(et, t);
+            if constexpr (kTurn)
+                acc += R.total(t & 63);
             epi.template apply_n<true>(v, w, (ZXA_CONST double *)(tphase + tile * Epi<kC64>::kStride), t);
+        }
+        if constexpr (kTurn)
+        {
+            adj_tile<kC64, kL1, kL2>(v, w, lds, G + 1, t, R);
+            acc2 += R.total(t & 63);
         }
         store_tile<kC64>(v, pp, base ^ toff, G);
         store_tile<kC64>(w, pl, base ^ toff, G);
-        acc += R.total(t & 63);
+        if constexpr (!kTurn)
+            acc += R.total(t & 63);
         base = next_base(base, P);
     }
-    partial[(size_t(blockIdx.x) * kWavesPerTile + (t >> 6)) * 64 + (t & 63)] = acc;
+    const size_t row = (size_t(blockIdx.x) * kWavesPerTile + (t >> 6)) * 64 + (t & 63);
+    partial[row] = acc;
+    if constexpr (kTurn)
+        partial[size_t(gridDim.x) * kWavesPerTile * 64 + row] = acc2;
 }
 
 // Sums rows [0, nrows) of 64 lane accumulators in a fixed order, then adds
 // every gradient entry into grads[param] (param < nparams) in entry order, so
-// that entries of one pass sharing a parameter never race.
+// that entries of one pass sharing a parameter never race.  One workgroup,
+// bound by the loads it has in flight: 16 waves of eight rows each, and the
+// entries at once (4 waves of four and the entries one by one took 43 us for
+// 2048 rows and 7 for 64, 20 and 6 now).
+constexpr int kCollectWaves = 16;
+constexpr int kCollectRows = 8;
 __device__ __forceinline__ void collect_rows(const double *__restrict__ partial, uint64_t nrows,
                                              const TGrad *__restrict__ tg, int64_t nparams, double *__restrict__ grads)
 {
-    static_assert(kWavesPerTile == 4, "four row groups");
-    __shared__ double part[kWavesPerTile][64];
+    __shared__ double part[kCollectWaves][64];
     __shared__ double tot[64];
     const int lane = threadIdx.x & 63;
     const int q = threadIdx.x >> 6;
-    // four independent partial sums per thread (loads in flight), in a fixed
-    // order: deterministic
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+    double s[kCollectRows] = {};
     uint64_t r = q;
-    for (; r + 3 * kWavesPerTile < nrows; r += 4 * kWavesPerTile)
-    {
-        s0 += partial[r * 64 + lane];
-        s1 += partial[(r + kWavesPerTile) * 64 + lane];
-        s2 += partial[(r + 2 * kWavesPerTile) * 64 + lane];
-        s3 += partial[(r + 3 * kWavesPerTile) * 64 + lane];
-    }
-    for (; r < nrows; r += kWavesPerTile)
-        s0 += partial[r * 64 + lane];
-    part[q][lane] = (s0 + s1) + (s2 + s3);
+    for (; r + (kCollectRows - 1) * kCollectWaves < nrows; r += kCollectRows * kCollectWaves)
+#pragma unroll
+        for (int k = 0; k < kCollectRows; k++)
+            s[k] += partial[(r + k * kCollectWaves) * 64 + lane];
+    for (; r < nrows; r += kCollectWaves)
+        s[0] += partial[r * 64 + lane];
+#pragma unroll
+    for (int k = kCollectRows / 2; k > 0; k /= 2)
+#pragma unroll
+        for (int l = 0; l < k; l++)
+            s[l] += s[l + k];
+    part[q][lane] = s[0];
     __syncthreads();
     if (threadIdx.x < 64)
-        tot[lane] = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
-    __syncthreads();
-    if (threadIdx.x == 0)
     {
-        for (int a = 0; a < kAccs; a++)
+        double a = part[0][lane];
+#pragma unroll
+        for (int k = 1; k < kCollectWaves; k++)
+            a += part[k][lane];
+        tot[lane] = a;
+    }
+    __syncthreads();
+    __shared__ double val[kAccs];
+    __shared__ int32_t at[kAccs];
+    const int a = threadIdx.x;
+    if (a < kAccs)
+    {
+        const TGrad g = tg[a];
+        val[a] = g.c[0] * tot[g.lane[0] & 63] + g.c[1] * tot[g.lane[1] & 63] + g.c[2] * tot[g.lane[2] & 63];
+        at[a] = g.param < nparams ? g.param : -1;
+    }
+    __syncthreads();
+    if (a < kAccs && at[a] >= 0)
+    {
+        // the parameter's first entry adds them all
+        bool first = true;
+        for (int k = 0; k < a; k++)
+            first = first && at[k] != at[a];
+        if (first)
         {
-            const TGrad &g = tg[a];
-            if (g.param < 0 || g.param >= nparams)
-                continue;
-            grads[g.param] += g.c[0] * tot[g.lane[0] & 63] + g.c[1] * tot[g.lane[1] & 63] +
-                              g.c[2] * tot[g.lane[2] & 63];
+            double x = grads[at[a]];
+            for (int k = a; k < kAccs; k++)
+                x += at[k] == at[a] ? val[k] : 0.0;
+            grads[at[a]] = x;
         }
     }
 }
 
-__global__ __launch_bounds__(kThreads) void adj_collect_kernel(const double *__restrict__ partial, uint64_t nrows,
+// rounds: sets of nrows rows and kAccs entries, one after the other (they may
+// share parameters).
+__global__ __launch_bounds__(64 * kCollectWaves) void adj_collect_kernel(const double *__restrict__ partial, uint64_t nrows,
                                                                const TGrad *__restrict__ tg, int64_t nparams,
-                                                               double *__restrict__ grads)
+                                                               double *__restrict__ grads, int rounds)
 {
-    collect_rows(partial, nrows, tg, nparams, grads);
+    for (int k = 0; k < rounds; k++)
+    {
+        collect_rows(partial + k * nrows * 64, nrows, tg + k * kAccs, nparams, grads);
+        __syncthreads();
+    }
 }
 
 __device__ __forceinline__ cd cis(double a)
@@ -3083,11 +3134,26 @@ int run_tile_pass(Ctx &ctx, void *state, int prec, unsigned n, const std::vector
     return ctx.ring.done(ctx.stream);
 }
 
-template <bool kC64, bool kL1, bool kL2, bool kDiag>
+template <bool kC64>
+int launch_turn(Ctx &ctx, void *state, const TPass &P0, bool l1, bool l2, const TTab *tab, const double *ttab,
+                const double *tphase)
+{
+    auto k = l1 && l2 ? tile_kernel<kC64, true, true, true, false, false, false, true>
+             : l1     ? tile_kernel<kC64, true, false, true, false, false, false, true>
+             : l2     ? tile_kernel<kC64, false, true, true, false, false, false, true>
+                      : tile_kernel<kC64, false, false, true, false, false, false, true>;
+    const int grid = persistent_grid(ctx, k, P0.ntiles);
+    TPass P = P0;
+    P.gstep = deposit(uint64_t(grid), P.sorted);
+    hipLaunchKernelGGL(k, dim3(grid), dim3(kThreads), 0, ctx.stream, state, P, tab, ttab, tphase);
+    return hip_check(hipGetLastError(), "turn pass launch");
+}
+
+template <bool kC64, bool kL1, bool kL2, bool kDiag, bool kTurn>
 int launch_adj_t(Ctx &ctx, void *psi, void *lam, const TPass &P0, const TTab *tab, const double *ttab,
                  const double *tphase, double *partial, int *nwaves)
 {
-    auto k = adj_kernel<kC64, kL1, kL2, kDiag>;
+    auto k = adj_kernel<kC64, kL1, kL2, kDiag, kTurn>;
     const int grid = persistent_grid(ctx, k, P0.ntiles);
     // the partial buffer holds *nwaves (on entry: its capacity in waves)
     if (grid * (kThreads / 64) > *nwaves)
@@ -3102,17 +3168,17 @@ int launch_adj_t(Ctx &ctx, void *psi, void *lam, const TPass &P0, const TTab *ta
     return hip_check(hipGetLastError(), "adj_kernel launch");
 }
 
-template <bool kC64, bool kDiag>
+template <bool kC64, bool kDiag, bool kTurn = false>
 int launch_adj_l(Ctx &ctx, void *psi, void *lam, const TPass &P, bool l1, bool l2, const TTab *tab,
                  const double *ttab, const double *tphase, double *partial, int *nwaves)
 {
     if (l1 && l2)
-        return launch_adj_t<kC64, true, true, kDiag>(ctx, psi, lam, P, tab, ttab, tphase, partial, nwaves);
+        return launch_adj_t<kC64, true, true, kDiag, kTurn>(ctx, psi, lam, P, tab, ttab, tphase, partial, nwaves);
     if (l1)
-        return launch_adj_t<kC64, true, false, kDiag>(ctx, psi, lam, P, tab, ttab, tphase, partial, nwaves);
+        return launch_adj_t<kC64, true, false, kDiag, kTurn>(ctx, psi, lam, P, tab, ttab, tphase, partial, nwaves);
     if (l2)
-        return launch_adj_t<kC64, false, true, kDiag>(ctx, psi, lam, P, tab, ttab, tphase, partial, nwaves);
-    return launch_adj_t<kC64, false, false, kDiag>(ctx, psi, lam, P, tab, ttab, tphase, partial, nwaves);
+        return launch_adj_t<kC64, false, true, kDiag, kTurn>(ctx, psi, lam, P, tab, ttab, tphase, partial, nwaves);
+    return launch_adj_t<kC64, false, false, kDiag, kTurn>(ctx, psi, lam, P, tab, ttab, tphase, partial, nwaves);
 }
 
 // Gradient entries of one target in slot `slot` (out: kAccs entries).  The
@@ -3161,6 +3227,15 @@ int grad_entries(bool c64, int slot, const AdjTarget &tg, size_t nparams, TGrad 
     return OK;
 }
 
+void set_matrix(TGate &g, const double *u)
+{
+    for (int k = 0; k < 8; k++)
+    {
+        g.u[k] = u[k];
+        g.uf[k] = float(u[k]);
+    }
+}
+
 void clear_grads(TGrad *g)
 {
     for (int a = 0; a < kAccs; a++)
@@ -3188,6 +3263,8 @@ struct BItem
     uint64_t tphase;  // epilogue per-tile factors (one identity row: no window)
     uint64_t tstride; // doubles per tile in tphase; 0: no window
     uint64_t partial; // adjoint: per tile and wave, a row of 64 lane sums
+    uint64_t tab2;    // TTab of a second round of gates after the window (0: none)
+    uint64_t partial2;
     uint32_t ub[kUnitBits];
     uint32_t sorted[kUnitBits];
 };
@@ -3240,27 +3317,20 @@ __device__ __forceinline__ void batch_store(const typename UnitT<kC64>::T (&v)[k
     store_tile<kC64>(v, reinterpret_cast<T *>(I.psi), base ^ thr_off<0>(t, P), (ZXA_CONST TTab *)I.tab);
 }
 
-// Gates and transposes of one forward tile, then the item's window (tphase
-// set) with the per-thread table e loaded before the tile's work.
+// One round of gates of a forward tile.
 template <bool kC64, bool kL1, bool kL2>
-__device__ __forceinline__ void batch_work(typename UnitT<kC64>::T (&v)[kRegs], typename UnitT<kC64>::T *lds,
-                                           ZXA_CONST BItem &I, uint64_t g, int t, const Epi<kC64> &e)
+__device__ __forceinline__ void batch_round(typename UnitT<kC64>::T (&v)[kRegs], typename UnitT<kC64>::T *lds,
+                                            const TPass &P, ZXA_CONST TTab *G, int t)
 {
-    TPass P;
-    batch_pass(I, P);
-    const uint64_t local = g - I.first;
-    const uint64_t base = deposit(local, P.sorted);
-    const uint64_t toff = thr_off<0>(t, P);
-    ZXA_CONST TTab *G = (ZXA_CONST TTab *)I.tab;
-    apply_layout<kC64, false, 0>(v, P, G, base, toff);
+    apply_layout<kC64, false, 0>(v, P, G, 0, 0);
     if constexpr (kL1)
     {
         transpose<kC64, 0, 1>(v, lds, t);
-        apply_layout<kC64, false, 1>(v, P, G, base, toff);
+        apply_layout<kC64, false, 1>(v, P, G, 0, 0);
         if constexpr (kL2)
         {
             transpose<kC64, 1, 2>(v, lds, t);
-            apply_layout<kC64, false, 2>(v, P, G, base, toff);
+            apply_layout<kC64, false, 2>(v, P, G, 0, 0);
             transpose<kC64, 2, 0>(v, lds, t);
         }
         else
@@ -3271,11 +3341,26 @@ __device__ __forceinline__ void batch_work(typename UnitT<kC64>::T (&v)[kRegs], 
     else if constexpr (kL2)
     {
         transpose<kC64, 0, 2>(v, lds, t);
-        apply_layout<kC64, false, 2>(v, P, G, base, toff);
+        apply_layout<kC64, false, 2>(v, P, G, 0, 0);
         transpose<kC64, 2, 0>(v, lds, t);
     }
-    if (I.tstride != 0)
+}
+
+// Gates of one forward tile, then the item's window (tphase set) with the
+// per-thread table e loaded before the tile's work, then (kTurn) the second
+// round's gates.
+template <bool kC64, bool kL1, bool kL2, bool kTurn>
+__device__ __forceinline__ void batch_work(typename UnitT<kC64>::T (&v)[kRegs], typename UnitT<kC64>::T *lds,
+                                           ZXA_CONST BItem &I, uint64_t g, int t, const Epi<kC64> &e)
+{
+    TPass P;
+    batch_pass(I, P);
+    const uint64_t local = g - I.first;
+    batch_round<kC64, kL1, kL2>(v, lds, P, (ZXA_CONST TTab *)I.tab, t);
+    if (kTurn || I.tstride != 0)
         e.apply(v, (ZXA_CONST double *)(reinterpret_cast<const double *>(I.tphase) + local * Epi<kC64>::kStride), t);
+    if constexpr (kTurn)
+        batch_round<kC64, kL1, kL2>(v, lds, P, (ZXA_CONST TTab *)I.tab2, t);
 }
 
 // Forward passes of many states, pipelined as tile_kernel: two register
@@ -3286,7 +3371,7 @@ __device__ __forceinline__ void batch_work(typename UnitT<kC64>::T (&v)[kRegs], 
 // loads are unconditional and issued before the prefetch: waiting for them
 // never waits for the prefetched tile.  Past the workgroup's last tile the
 // prefetch re-reads the current one.
-template <bool kC64, bool kL1, bool kL2>
+template <bool kC64, bool kL1, bool kL2, bool kTurn>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void batch_fwd_kernel(
     const BItem *__restrict__ items, int nitems, uint64_t total)
 {
@@ -3308,7 +3393,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     int i1 = m1 ? batch_find(IT, nitems, g1) : i0;
     uint64_t h1 = m1 ? g1 : g0;
     batch_load<kC64>(b, IT[i1], h1, t);
-    batch_work<kC64, kL1, kL2>(a, lds, IT[i0], g0, t, e);
+    batch_work<kC64, kL1, kL2, kTurn>(a, lds, IT[i0], g0, t, e);
     for (;;)
     {
         batch_store<kC64>(a, IT[i0], g0, t);
@@ -3320,7 +3405,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         const uint64_t h2 = m2 ? g2 : g1;
         e.init(reinterpret_cast<const double *>(IT[i1].ttab), t);
         batch_load<kC64>(a, IT[i2], h2, t);
-        batch_work<kC64, kL1, kL2>(b, lds, IT[i1], g1, t, e);
+        batch_work<kC64, kL1, kL2, kTurn>(b, lds, IT[i1], g1, t, e);
 
         batch_store<kC64>(b, IT[i1], g1, t);
         if (!m2)
@@ -3331,7 +3416,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         const uint64_t h3 = m3 ? g3 : g2;
         e.init(reinterpret_cast<const double *>(IT[i2].ttab), t);
         batch_load<kC64>(b, IT[i3], h3, t);
-        batch_work<kC64, kL1, kL2>(a, lds, IT[i2], g2, t, e);
+        batch_work<kC64, kL1, kL2, kTurn>(a, lds, IT[i2], g2, t, e);
 
         g0 = g2;
         i0 = i2;
@@ -3344,7 +3429,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
 // Adjoint passes of many states, one tile per step (two states per tile
 // leave no registers for a second buffer).  kL1 / kL2: the launch's items use
 // layout 1 / 2 (any of them); items that do not get identity matrices there.
-template <bool kC64, bool kL1, bool kL2>
+template <bool kC64, bool kL1, bool kL2, bool kTurn>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void batch_adj_kernel(
     const BItem *__restrict__ items, int nitems, uint64_t total)
 {
@@ -3370,54 +3455,53 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
         load_tile<kC64>(v, pp, base ^ toff, G);
         load_tile<kC64>(w, pl, base ^ toff, G);
         AdjRest<kC64> R;
+        double *rows = reinterpret_cast<double *>(I.partial);
+        const size_t row = (local * kWavesPerTile + (t >> 6)) * 64 + lane;
         adj_tile<kC64, kL1, kL2>(v, w, lds, G, t, R);
+        if constexpr (kTurn)
+            rows[row] = R.total(lane);
         // unconditional (identity tables where the item has no window): a
-        // branch around the epilogue made the compiler spill about 90 VGPRs.
-        // The per-thread factors are read here, not held across the tile.
+        // branch around the epilogue made the compiler spill about 90 VGPRs
+        // (so did a loop over the rounds).  The per-thread factors are read
+        // here, not held across the tile.
         const double *et = reinterpret_cast<const double *>(I.ttab);
         asm volatile("" : "+s"(et));
         Epi<kC64> epi;
         epi.init(et, t);
         epi.template apply_n<true>(
             v, w, (ZXA_CONST double *)(reinterpret_cast<const double *>(I.tphase) + local * I.tstride), t);
-        store_tile<kC64>(v, pp, base ^ toff, G);
-        store_tile<kC64>(w, pl, base ^ toff, G);
-        reinterpret_cast<double *>(I.partial)[(local * kWavesPerTile + (t >> 6)) * 64 + lane] = R.total(lane);
-    }
-}
-
-template <bool kC64, bool kAdj>
-auto batch_kernel_for(bool l1, bool l2)
-{
-    if constexpr (kAdj)
-    {
-        if (l1 && l2)
-            return batch_adj_kernel<kC64, true, true>;
-        if (l1)
-            return batch_adj_kernel<kC64, true, false>;
-        if (l2)
-            return batch_adj_kernel<kC64, false, true>;
-        return batch_adj_kernel<kC64, false, false>;
-    }
-    else
-    {
-        if (l1 && l2)
-            return batch_fwd_kernel<kC64, true, true>;
-        if (l1)
-            return batch_fwd_kernel<kC64, true, false>;
-        if (l2)
-            return batch_fwd_kernel<kC64, false, true>;
-        return batch_fwd_kernel<kC64, false, false>;
+        if constexpr (kTurn)
+        {
+            adj_tile<kC64, kL1, kL2>(v, w, lds, (ZXA_CONST TTab *)I.tab2, t, R);
+            rows = reinterpret_cast<double *>(I.partial2);
+        }
+        store_tile<kC64>(v, pp, base ^ toff, (ZXA_CONST TTab *)I.tab);
+        store_tile<kC64>(w, pl, base ^ toff, (ZXA_CONST TTab *)I.tab);
+        rows[row] = R.total(lane);
     }
 }
 
 using BatchKernel = void (*)(const BItem *, int, uint64_t);
 
-BatchKernel batch_kernel(bool c64, bool adj, bool l1, bool l2)
+template <bool kC64, bool kTurn>
+BatchKernel batch_kernel_for(bool adj, bool l1, bool l2)
+{
+    if (adj)
+        return l1 && l2 ? batch_adj_kernel<kC64, true, true, kTurn>
+               : l1     ? batch_adj_kernel<kC64, true, false, kTurn>
+               : l2     ? batch_adj_kernel<kC64, false, true, kTurn>
+                        : batch_adj_kernel<kC64, false, false, kTurn>;
+    return l1 && l2 ? batch_fwd_kernel<kC64, true, true, kTurn>
+           : l1     ? batch_fwd_kernel<kC64, true, false, kTurn>
+           : l2     ? batch_fwd_kernel<kC64, false, true, kTurn>
+                    : batch_fwd_kernel<kC64, false, false, kTurn>;
+}
+
+BatchKernel batch_kernel(bool c64, bool adj, const BatchLaunch::Part &p)
 {
     if (c64)
-        return adj ? batch_kernel_for<true, true>(l1, l2) : batch_kernel_for<true, false>(l1, l2);
-    return adj ? batch_kernel_for<false, true>(l1, l2) : batch_kernel_for<false, false>(l1, l2);
+        return p.turn ? batch_kernel_for<true, true>(adj, p.l1, p.l2) : batch_kernel_for<true, false>(adj, p.l1, p.l2);
+    return p.turn ? batch_kernel_for<false, true>(adj, p.l1, p.l2) : batch_kernel_for<false, false>(adj, p.l1, p.l2);
 }
 
 // Per item (one workgroup each): the rows of its tiles and waves summed in a
@@ -3429,13 +3513,19 @@ struct BCollect
     uint64_t grad;    // TGrad[kAccs]
     uint64_t grads;   // double*
     int64_t nparams;  // length of grads
+    uint64_t partial2, grad2; // the second round's (0: none), after the first's
 };
 
-__global__ __launch_bounds__(kThreads) void batch_collect_kernel(const BCollect *__restrict__ items)
+__global__ __launch_bounds__(64 * kCollectWaves) void batch_collect_kernel(const BCollect *__restrict__ items)
 {
     const BCollect &I = items[blockIdx.x];
     collect_rows(reinterpret_cast<const double *>(I.partial), I.ntiles * kWavesPerTile,
                  reinterpret_cast<const TGrad *>(I.grad), I.nparams, reinterpret_cast<double *>(I.grads));
+    if (!I.partial2)
+        return;
+    __syncthreads();
+    collect_rows(reinterpret_cast<const double *>(I.partial2), I.ntiles * kWavesPerTile,
+                 reinterpret_cast<const TGrad *>(I.grad2), I.nparams, reinterpret_cast<double *>(I.grads));
 }
 
 } // namespace
@@ -3877,6 +3967,68 @@ int fused_pass_apply(Ctx &ctx, void *state, int prec, unsigned n, const U3Gate *
     return run_tile_pass(ctx, state, prec, n, gs, diag, ndiag, geometry, fans, fresh);
 }
 
+int turn_pass_apply(Ctx &ctx, void *state, int prec, unsigned n, const U3Gate *gates, size_t ngates,
+                    const DiagGate *diag, size_t ndiag, const U3Gate *gates2, size_t ngates2, int geometry)
+{
+    if (n < tile_min_bits(prec) || n > 40 || ndiag == 0 || !window_is_polynomial(n, diag, ndiag))
+    {
+        set_error("turn pass: state narrower than a tile, or a window that is no phase polynomial");
+        return EINVAL_;
+    }
+    const U3Gate *ts[2] = {gates, gates2};
+    const size_t nts[2] = {ngates, ngates2};
+    std::vector<SingleGate> gs;
+    for (int r = 0; r < 2; r++)
+        for (size_t i = 0; i < nts[r]; i++)
+        {
+            const U3Gate &g = ts[r][i];
+            if (g.delta == 0 || (g.delta & (g.delta - 1)) != 0 || g.packed_sel != g.delta || (g.delta >> n) != 0)
+            {
+                set_error("turn pass: gate is not a single-bit U3");
+                return EINVAL_;
+            }
+            for (size_t j = 0; j < i; j++)
+                if (ts[r][j].delta == g.delta)
+                {
+                    set_error("turn pass: two gates of a round on one target");
+                    return EINVAL_;
+                }
+            const unsigned t = unsigned(__builtin_ctzll(g.delta));
+            if (std::none_of(gs.begin(), gs.end(), [&](const SingleGate &o) { return o.target == t; }))
+                gs.push_back({t, &g});
+        }
+    Plan pl;
+    if (!plan_tile(prec, n, gs, pl, geometry))
+    {
+        set_error("turn pass: more targets than the tile has slots");
+        return EINVAL_;
+    }
+    TPass P;
+    TTab G[2];
+    bool use[3];
+    fill_pass(prec, n, pl, P, G[0], use);
+    G[1] = G[0];
+    for (int r = 0; r < 2; r++)
+        for (size_t i = 0; i < nts[r]; i++)
+            for (size_t k = 0; k < gs.size(); k++)
+                if (gs[k].g->delta == ts[r][i].delta)
+                    set_matrix(G[r].g[pl.slot[k]], ts[r][i].u);
+    const double *ttab = nullptr;
+    const double *tphase = nullptr;
+    PassBatch batch(ctx);
+    ZXA_TRY(batch.begin());
+    ZXA_TRY(setup_epilogue(ctx, prec, n, pl.ebit, diag, ndiag, P.ntiles, &ttab, &tphase, 8, batch.ph));
+    void *dtab = nullptr;
+    ZXA_TRY(ctx.ring.stage(G, sizeof(G), ctx.stream, &dtab));
+    ZXA_TRY(batch.run());
+    const TTab *tab = static_cast<const TTab *>(dtab);
+    ZXA_TRY(ctx.tic());
+    ZXA_TRY(prec == C64 ? launch_turn<true>(ctx, state, P, use[1], use[2], tab, ttab, tphase)
+                        : launch_turn<false>(ctx, state, P, use[1], use[2], tab, ttab, tphase));
+    ZXA_TRY(ctx.toc(F_FUSED, 2ull * (uint64_t(1) << n) * elem_bytes(prec)));
+    return ctx.ring.done(ctx.stream);
+}
+
 } // namespace zxa
 
 namespace zxa
@@ -3884,7 +4036,7 @@ namespace zxa
 
 int adjoint_pass_apply(Ctx &ctx, void *psi, void *lam, int prec, unsigned n, const AdjTarget *targets,
                        size_t ntargets, const DiagGate *diag, size_t ndiag, double *dgrads, size_t nparams,
-                       int geometry)
+                       int geometry, const AdjTarget *targets2, size_t ntargets2)
 {
     const bool c64 = prec == C64;
     if (n < tile_min_bits(prec) || n > 40)
@@ -3897,26 +4049,42 @@ int adjoint_pass_apply(Ctx &ctx, void *psi, void *lam, int prec, unsigned n, con
         set_error("adjoint pass: diagonal window is not a phase polynomial");
         return EINVAL_;
     }
-    std::vector<U3Gate> ug(ntargets);
-    std::vector<SingleGate> gs;
-    for (size_t i = 0; i < ntargets; i++)
+    const bool turn = ntargets2 > 0;
+    if (turn && ndiag == 0)
     {
-        const unsigned q = targets[i].target;
-        if (q >= n)
+        set_error("adjoint pass: two rounds need a window between them");
+        return EINVAL_;
+    }
+    // a tile for the targets of both rounds
+    const AdjTarget *ts[2] = {targets, targets2};
+    const size_t nts[2] = {ntargets, ntargets2};
+    U3Gate ug[64];
+    std::vector<SingleGate> gs;
+    uint64_t all = 0;
+    for (int r = 0; r < 2; r++)
+    {
+        uint64_t seen = 0;
+        for (size_t i = 0; i < nts[r]; i++)
         {
-            set_error("adjoint pass: target outside the state");
-            return EINVAL_;
-        }
-        for (size_t j = 0; j < i; j++)
-            if (targets[j].target == q)
+            const unsigned q = ts[r][i].target;
+            if (q >= n)
+            {
+                set_error("adjoint pass: target outside the state");
+                return EINVAL_;
+            }
+            const uint64_t bit = uint64_t(1) << q;
+            if (seen & bit)
             {
                 set_error("adjoint pass: two entries on one target");
                 return EINVAL_;
             }
-        ug[i].packed_sel = uint64_t(1) << q;
-        ug[i].delta = uint64_t(1) << q;
-        std::memcpy(ug[i].u, targets[i].m, sizeof(ug[i].u));
-        gs.push_back({q, &ug[i]});
+            seen |= bit;
+            ug[q].packed_sel = bit;
+            ug[q].delta = bit;
+            if (!(all & bit))
+                gs.push_back({q, &ug[q]});
+            all |= bit;
+        }
     }
     Plan pl;
     if (!plan_tile(prec, n, gs, pl, geometry))
@@ -3925,21 +4093,26 @@ int adjoint_pass_apply(Ctx &ctx, void *psi, void *lam, int prec, unsigned n, con
         return EINVAL_;
     }
     TPass P;
-    TTab G;
+    TTab G[2];
     bool use[3];
-    fill_pass(prec, n, pl, P, G, use);
-    TGrad tg[kAccs];
-    clear_grads(tg);
-    for (size_t i = 0; i < ntargets; i++)
+    fill_pass(prec, n, pl, P, G[0], use);
+    G[1] = G[0];
+    TGrad tg[2 * kAccs];
+    for (int r = 0; r < 2; r++)
     {
-        const int slot = pl.slot[i];
-        for (int k = 0; k < 8; k++)
+        clear_grads(tg + r * kAccs);
+        for (size_t i = 0; i < nts[r]; i++)
         {
-            G.g[slot].u[k] = targets[i].m[k];
-            G.g[slot].uf[k] = float(targets[i].m[k]);
+            const AdjTarget &t = ts[r][i];
+            size_t k = 0;
+            while (gs[k].target != t.target)
+                k++;
+            const int slot = pl.slot[k];
+            set_matrix(G[r].g[slot], t.m);
+            ZXA_TRY(grad_entries(c64, slot, t, nparams, tg + r * kAccs));
         }
-        ZXA_TRY(grad_entries(c64, slot, targets[i], nparams, tg));
     }
+    const size_t rounds = turn ? 2 : 1;
     const double *ttab = nullptr;
     const double *tphase = nullptr;
     PassBatch batch(ctx);
@@ -3947,19 +4120,24 @@ int adjoint_pass_apply(Ctx &ctx, void *psi, void *lam, int prec, unsigned n, con
     if (ndiag > 0)
         ZXA_TRY(setup_epilogue(ctx, prec, n, pl.ebit, diag, ndiag, P.ntiles, &ttab, &tphase, 8, batch.ph));
     void *dtab = nullptr, *dgr = nullptr;
-    ZXA_TRY(ctx.ring.stage(&G, sizeof(G), ctx.stream, &dtab));
-    ZXA_TRY(ctx.ring.stage(tg, sizeof(tg), ctx.stream, &dgr));
+    ZXA_TRY(ctx.ring.stage(G, rounds * sizeof(TTab), ctx.stream, &dtab));
+    ZXA_TRY(ctx.ring.stage(tg, rounds * kAccs * sizeof(TGrad), ctx.stream, &dgr));
     ZXA_TRY(batch.run());
     // per-wave rows of 64 lane accumulators: at most 8 workgroups per CU
-    const size_t maxw = size_t(8) * size_t(ctx.num_cus > 0 ? ctx.num_cus : 256) * kWavesPerTile;
-    ZXA_TRY(ctx.scratch_f.ensure(maxw * 64 * sizeof(double)));
+    // (allocated for two rounds from the start)
+    const size_t maxw = std::min<size_t>(P.ntiles, size_t(8) * size_t(ctx.num_cus > 0 ? ctx.num_cus : 256)) * kWavesPerTile;
+    ZXA_TRY(ctx.scratch_f.ensure(2 * maxw * 64 * sizeof(double)));
     double *partial = static_cast<double *>(ctx.scratch_f.ptr);
     const TTab *tab = static_cast<const TTab *>(dtab);
     const uint64_t bytes = 4ull * (uint64_t(1) << n) * elem_bytes(prec);
     int nwaves = int(maxw);
     ZXA_TRY(ctx.tic());
     int rc;
-    if (c64)
+    if (turn)
+        rc = c64 ? launch_adj_l<true, true, true>(ctx, psi, lam, P, use[1], use[2], tab, ttab, tphase, partial, &nwaves)
+                 : launch_adj_l<false, true, true>(ctx, psi, lam, P, use[1], use[2], tab, ttab, tphase, partial,
+                                                   &nwaves);
+    else if (c64)
         rc = ndiag ? launch_adj_l<true, true>(ctx, psi, lam, P, use[1], use[2], tab, ttab, tphase, partial, &nwaves)
                    : launch_adj_l<true, false>(ctx, psi, lam, P, use[1], use[2], tab, ttab, tphase, partial, &nwaves);
     else
@@ -3968,8 +4146,8 @@ int adjoint_pass_apply(Ctx &ctx, void *psi, void *lam, int prec, unsigned n, con
                                                 &nwaves);
     ZXA_TRY(rc);
     ZXA_TRY(ctx.toc(F_ADJ, bytes));
-    hipLaunchKernelGGL(adj_collect_kernel, dim3(1), dim3(kThreads), 0, ctx.stream, partial, uint64_t(nwaves),
-                       static_cast<const TGrad *>(dgr), int64_t(nparams), dgrads);
+    hipLaunchKernelGGL(adj_collect_kernel, dim3(1), dim3(64 * kCollectWaves), 0, ctx.stream, partial, uint64_t(nwaves),
+                       static_cast<const TGrad *>(dgr), int64_t(nparams), dgrads, int(rounds));
     ZXA_HIP(hipGetLastError());
     return ctx.ring.done(ctx.stream);
 }
@@ -4012,13 +4190,25 @@ int batch_prepare(Ctx &ctx, int prec, bool adj, const std::vector<BatchPassSpec>
     b.prec = prec;
     b.adj = adj;
     b.nitems = specs.size();
-    b.slots.assign(specs.size(), {});
+    // tables: every item's first round, then the second rounds
+    size_t ntabs = specs.size();
+    for (int r = 0; r < 2; r++)
+    {
+        b.slots[r].assign(specs.size(), {});
+        b.tab[r].assign(specs.size(), 0);
+    }
+    for (size_t i = 0; i < specs.size(); i++)
+    {
+        b.tab[0][i] = i;
+        if (!specs[i].targets2.empty())
+            b.tab[1][i] = ntabs++;
+    }
     if (specs.empty())
         return OK;
     std::vector<BItem> items(specs.size());
-    std::vector<TTab> tabs(specs.size());
-    std::vector<TGrad> grads(adj ? specs.size() * kAccs : 0);
-    for (size_t i = 0; i < specs.size() && adj; i++)
+    std::vector<TTab> tabs(ntabs);
+    std::vector<TGrad> grads(adj ? ntabs * kAccs : 0);
+    for (size_t i = 0; i < ntabs && adj; i++)
         clear_grads(&grads[i * kAccs]);
     b.nparams.assign(specs.size(), 0);
     // epilogue tables: per item, per-thread table then per-tile factors.  The
@@ -4030,8 +4220,9 @@ int batch_prepare(Ctx &ctx, int prec, bool adj, const std::vector<BatchPassSpec>
     const size_t stride = 2 * (8 + (size_t(1) << nb));
     std::vector<size_t> epi_off(specs.size(), 0), epi_tt(specs.size(), 0);
     size_t epi_bytes = (ttab_doubles + stride) * sizeof(double);
-    uint64_t first = 0, partial_doubles = 0;
+    uint64_t partial_doubles = 0;
     std::vector<Plan> plans(specs.size());
+    std::vector<int> part_of(specs.size(), 0);
     for (size_t i = 0; i < specs.size(); i++)
     {
         const BatchPassSpec &sp = specs[i];
@@ -4040,12 +4231,16 @@ int batch_prepare(Ctx &ctx, int prec, bool adj, const std::vector<BatchPassSpec>
             set_error("batch: state narrower than a tile");
             return EINVAL_;
         }
-        std::vector<U3Gate> ug(sp.targets.size());
+        std::vector<unsigned> ts = sp.targets;
+        for (unsigned q : sp.targets2)
+            if (std::find(ts.begin(), ts.end(), q) == ts.end())
+                ts.push_back(q);
+        std::vector<U3Gate> ug(ts.size());
         std::vector<SingleGate> gs;
-        for (size_t k = 0; k < sp.targets.size(); k++)
+        for (size_t k = 0; k < ts.size(); k++)
         {
-            ug[k].packed_sel = ug[k].delta = uint64_t(1) << sp.targets[k];
-            gs.push_back({sp.targets[k], &ug[k]});
+            ug[k].packed_sel = ug[k].delta = uint64_t(1) << ts[k];
+            gs.push_back({ts[k], &ug[k]});
         }
         if (!plan_tile(prec, sp.n, gs, plans[i], sp.geometry))
         {
@@ -4055,13 +4250,33 @@ int batch_prepare(Ctx &ctx, int prec, bool adj, const std::vector<BatchPassSpec>
         TPass P;
         bool use[3];
         fill_pass(prec, sp.n, plans[i], P, tabs[i], use);
-        b.l1 = b.l1 || use[1];
-        b.l2 = b.l2 || use[2];
-        b.slots[i] = plans[i].slot;
+        for (int r = 0; r < 2; r++)
+            for (unsigned q : r ? sp.targets2 : sp.targets)
+                b.slots[r][i].push_back(plans[i].slot[size_t(std::find(ts.begin(), ts.end(), q) - ts.begin())]);
         BItem &it = items[i];
         std::memset(&it, 0, sizeof(it));
-        it.first = first;
+        // its part: items of two rounds, and items without targets in
+        // layout 2, run kernels of their own (a kernel applies every layout
+        // that any of its items uses)
+        const int part = (sp.targets2.empty() ? 0 : 2) + (use[2] ? 1 : 0);
+        part_of[i] = part;
+        BatchLaunch::Part &pt = b.parts[part];
+        pt.turn = !sp.targets2.empty();
+        pt.l1 = pt.l1 || use[1];
+        pt.l2 = use[2];
+        if (!sp.targets2.empty())
+        {
+            tabs[b.tab[1][i]] = tabs[i];
+            if (sp.window.empty())
+            {
+                set_error("batch: two rounds need a window between them");
+                return EINVAL_;
+            }
+        }
+        it.first = pt.total_tiles;
         it.ntiles = P.ntiles;
+        pt.total_tiles += P.ntiles;
+        pt.nitems++;
         it.psi = reinterpret_cast<uint64_t>(sp.psi);
         it.lam = reinterpret_cast<uint64_t>(sp.lam);
         for (int k = 0; k < kUnitBits; k++)
@@ -4069,11 +4284,13 @@ int batch_prepare(Ctx &ctx, int prec, bool adj, const std::vector<BatchPassSpec>
             it.ub[k] = P.ub[k];
             it.sorted[k] = P.sorted[k];
         }
-        first += P.ntiles;
         if (adj)
         {
             it.partial = partial_doubles; // offset for now
             partial_doubles += P.ntiles * kWavesPerTile * 64;
+            it.partial2 = partial_doubles;
+            if (!sp.targets2.empty())
+                partial_doubles += P.ntiles * kWavesPerTile * 64;
             b.nparams[i] = sp.nparams;
         }
         if (!sp.window.empty())
@@ -4089,8 +4306,7 @@ int batch_prepare(Ctx &ctx, int prec, bool adj, const std::vector<BatchPassSpec>
             epi_bytes += P.ntiles * stride * sizeof(double);
         }
     }
-    b.total_tiles = first;
-    b.tab_bytes = specs.size() * sizeof(TTab);
+    b.tab_bytes = ntabs * sizeof(TTab);
     b.adj_bytes = grads.size() * sizeof(TGrad);
     char *dtabs = nullptr;
     ZXA_TRY(dmalloc(&dtabs, b.tab_bytes + b.adj_bytes));
@@ -4121,9 +4337,14 @@ int batch_prepare(Ctx &ctx, int prec, bool adj, const std::vector<BatchPassSpec>
     {
         BItem &it = items[i];
         it.tab = reinterpret_cast<uint64_t>(dtabs + i * sizeof(TTab));
-        if (adj)
-            it.partial = reinterpret_cast<uint64_t>(dpart + it.partial);
         const BatchPassSpec &sp = specs[i];
+        const bool turn = !sp.targets2.empty();
+        it.tab2 = turn ? reinterpret_cast<uint64_t>(dtabs + b.tab[1][i] * sizeof(TTab)) : 0;
+        if (adj)
+        {
+            it.partial = reinterpret_cast<uint64_t>(dpart + it.partial);
+            it.partial2 = turn ? reinterpret_cast<uint64_t>(dpart + it.partial2) : 0;
+        }
         it.ttab = reinterpret_cast<uint64_t>(depi);
         it.tphase = reinterpret_cast<uint64_t>(depi + ttab_doubles * sizeof(double));
         it.tstride = 0;
@@ -4149,8 +4370,17 @@ int batch_prepare(Ctx &ctx, int prec, bool adj, const std::vector<BatchPassSpec>
         it.tphase = reinterpret_cast<uint64_t>(depi + epi_off[i]);
         it.tstride = stride;
     }
-    ZXA_TRY(dmalloc(&b.d_items, items.size() * sizeof(BItem)));
-    ZXA_HIP(hipMemcpy(b.d_items, items.data(), items.size() * sizeof(BItem), hipMemcpyHostToDevice));
+    // the items, part by part
+    std::vector<BItem> ordered;
+    for (int k = 0; k < BatchLaunch::kParts; k++)
+    {
+        b.parts[k].first = ordered.size();
+        for (size_t i = 0; i < specs.size(); i++)
+            if (part_of[i] == k)
+                ordered.push_back(items[i]);
+    }
+    ZXA_TRY(dmalloc(&b.d_items, ordered.size() * sizeof(BItem)));
+    ZXA_HIP(hipMemcpy(b.d_items, ordered.data(), ordered.size() * sizeof(BItem), hipMemcpyHostToDevice));
     if (adj)
     {
         std::vector<BCollect> col(specs.size());
@@ -4161,43 +4391,36 @@ int batch_prepare(Ctx &ctx, int prec, bool adj, const std::vector<BatchPassSpec>
             col[i].grad = reinterpret_cast<uint64_t>(dtabs + b.tab_bytes + i * kAccs * sizeof(TGrad));
             col[i].grads = reinterpret_cast<uint64_t>(specs[i].grads);
             col[i].nparams = int64_t(specs[i].nparams);
+            col[i].partial2 = items[i].partial2;
+            col[i].grad2 = reinterpret_cast<uint64_t>(dtabs + b.tab_bytes + b.tab[1][i] * kAccs * sizeof(TGrad));
         }
         ZXA_TRY(dmalloc(&b.d_collect, col.size() * sizeof(BCollect)));
         ZXA_HIP(hipMemcpy(b.d_collect, col.data(), col.size() * sizeof(BCollect), hipMemcpyHostToDevice));
     }
-    b.grid = persistent_grid(ctx, batch_kernel(c64, adj, b.l1, b.l2), b.total_tiles);
+    for (BatchLaunch::Part &p : b.parts)
+        if (p.nitems)
+            p.grid = persistent_grid(ctx, batch_kernel(c64, adj, p), p.total_tiles);
     return OK;
 }
 
-void batch_set_gates(BatchLaunch &b, size_t item, const U3Gate *gates, size_t ngates)
+void batch_set_gates(BatchLaunch &b, size_t item, int round, const U3Gate *gates, size_t ngates)
 {
-    TTab *tab = reinterpret_cast<TTab *>(b.h_tables) + item;
-    for (size_t k = 0; k < ngates && k < b.slots[item].size(); k++)
-    {
-        TGate &tg = tab->g[b.slots[item][k]];
-        for (int i = 0; i < 8; i++)
-        {
-            tg.u[i] = gates[k].u[i];
-            tg.uf[i] = float(gates[k].u[i]);
-        }
-    }
+    TTab *tab = reinterpret_cast<TTab *>(b.h_tables) + b.tab[round][item];
+    const std::vector<int> &slots = b.slots[round][item];
+    for (size_t k = 0; k < ngates && k < slots.size(); k++)
+        set_matrix(tab->g[slots[k]], gates[k].u);
 }
 
-int batch_set_adjoint(BatchLaunch &b, size_t item, const AdjTarget *targets, size_t ntargets)
+int batch_set_adjoint(BatchLaunch &b, size_t item, int round, const AdjTarget *targets, size_t ntargets)
 {
-    TTab *tab = reinterpret_cast<TTab *>(b.h_tables) + item;
-    TGrad *gr = reinterpret_cast<TGrad *>(static_cast<char *>(b.h_tables) + b.tab_bytes) + item * kAccs;
+    TTab *tab = reinterpret_cast<TTab *>(b.h_tables) + b.tab[round][item];
+    TGrad *gr = reinterpret_cast<TGrad *>(static_cast<char *>(b.h_tables) + b.tab_bytes) + b.tab[round][item] * kAccs;
+    const std::vector<int> &slots = b.slots[round][item];
     clear_grads(gr);
-    for (size_t k = 0; k < ntargets && k < b.slots[item].size(); k++)
+    for (size_t k = 0; k < ntargets && k < slots.size(); k++)
     {
-        const int slot = b.slots[item][k];
-        TGate &tg = tab->g[slot];
-        for (int i = 0; i < 8; i++)
-        {
-            tg.u[i] = targets[k].m[i];
-            tg.uf[i] = float(targets[k].m[i]);
-        }
-        ZXA_TRY(grad_entries(b.prec == C64, slot, targets[k], b.nparams[item], gr));
+        set_matrix(tab->g[slots[k]], targets[k].m);
+        ZXA_TRY(grad_entries(b.prec == C64, slots[k], targets[k], b.nparams[item], gr));
     }
     return OK;
 }
@@ -4216,12 +4439,17 @@ int batch_launch(Ctx &ctx, BatchLaunch &b)
     if (!b.nitems)
         return OK;
     const bool c64 = b.prec == C64;
-    hipLaunchKernelGGL(batch_kernel(c64, b.adj, b.l1, b.l2), dim3(b.grid), dim3(kThreads), 0, ctx.stream, static_cast<const BItem *>(b.d_items),
-                       int(b.nitems), b.total_tiles);
-    ZXA_HIP(hipGetLastError());
+    for (const BatchLaunch::Part &p : b.parts)
+    {
+        if (!p.nitems)
+            continue;
+        hipLaunchKernelGGL(batch_kernel(c64, b.adj, p), dim3(p.grid), dim3(kThreads), 0, ctx.stream,
+                           static_cast<const BItem *>(b.d_items) + p.first, int(p.nitems), p.total_tiles);
+        ZXA_HIP(hipGetLastError());
+    }
     if (b.adj)
     {
-        hipLaunchKernelGGL(batch_collect_kernel, dim3(unsigned(b.nitems)), dim3(kThreads), 0, ctx.stream,
+        hipLaunchKernelGGL(batch_collect_kernel, dim3(unsigned(b.nitems)), dim3(64 * kCollectWaves), 0, ctx.stream,
                            static_cast<const BCollect *>(b.d_collect));
         ZXA_HIP(hipGetLastError());
     }
