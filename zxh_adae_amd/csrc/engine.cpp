@@ -311,20 +311,24 @@ int Sim::resize_reset(size_t M)
     used_bits_ = 0;
     if (policy_ == POLICY_FUSED)
     {
-        fresh_ = true;
-        fresh_elems_ = cap;
+        valid_ = 0;
         return OK;
     }
-    fresh_ = false;
+    valid_ = cap;
     return state_reset(ctx_, dstate_, prec_, cap);
 }
 
-int Sim::settle()
+int Sim::settle(size_t elems)
 {
-    if (!fresh_)
+    // (at least one 16-byte unit: what zero_fill continues from)
+    elems = std::min(std::max<size_t>(elems, 2), size_t(1) << M_);
+    if (valid_ >= elems)
         return OK;
-    fresh_ = false;
-    return state_reset(ctx_, dstate_, prec_, fresh_elems_);
+    const size_t from = valid_, size = elem_bytes(prec_);
+    valid_ = elems;
+    if (from == 0)
+        return state_reset(ctx_, dstate_, prec_, elems);
+    return zero_fill(ctx_, static_cast<char *>(dstate_) + from * size, (elems - from) * size);
 }
 
 int Sim::expand()
@@ -414,7 +418,9 @@ int Sim::flush_group()
 {
     if (exp_group_.empty())
         return OK;
-    ZXA_TRY(settle());
+    // an expansion reads the old bits' amplitudes only, and writes the others
+    ZXA_TRY(settle(size_t(1) << exp_base_));
+    valid_ = std::max(valid_, size_t(1) << (exp_base_ + exp_group_.size()));
     const int rc = u3_expand_group_apply(ctx_, dstate_, prec_, exp_base_, exp_group_.data(), exp_group_.size());
     exp_group_.clear();
     return rc;
@@ -448,10 +454,10 @@ int Sim::flush_pass()
     ZXA_TRY(flush_group());
     // the first pass after the reset forms |0...0> itself when it covers the
     // whole reset state (it resets the state where its kernel cannot)
-    const bool fresh = fresh_ && (size_t(1) << active_bits()) == fresh_elems_;
+    const bool fresh = valid_ == 0 && active_bits() == M_;
     if (!fresh)
         ZXA_TRY(settle());
-    fresh_ = false;
+    valid_ = std::max(valid_, size_t(1) << active_bits());
     int rc = fused_pass_apply(ctx_, dstate_, prec_, active_bits(), pass_u3_.data(), pass_u3_.size(),
                               pass_diag_.data(), pass_diag_.size(), -1,
                               pass_has_fan_ ? pass_fan_.data() : nullptr, fresh);
@@ -819,7 +825,7 @@ int Sim::execute()
     use_lds_ = policy_ == POLICY_FUSED && suits_lds();
     if (use_lds_)
     {
-        fresh_ = false; // the circuit's first run forms |0...0>
+        valid_ = size_t(1) << M_; // the circuit's first run forms |0...0>
         circuit_.begin(unsigned(M_), prec_);
     }
 
@@ -848,7 +854,9 @@ int Sim::execute()
     // sweeps and 39.2 ms with a flush at each such pair, three and 16.1 ms
     // without.)
     const bool stream = policy_ == POLICY_FUSED;
-    // expansions applied at once (u3_expand_group_apply)
+    // expansions applied at once (u3_expand_group_apply), in groups that end
+    // at M_, M_ - 4, ...: the last one, which writes the whole state, is full
+    // (25 qubits of complex128: 106 us, and 50 + 121 where a single bit came last)
     constexpr size_t kGroupMax = 4;
     std::vector<DiagGate> pre, post;
     std::vector<Acc> pend(N_);
@@ -1003,7 +1011,7 @@ int Sim::execute()
                 // the new bit is the top one and its half still zero
                 const bool top = eg.delta == uint64_t(1) << (active_bits() - 1);
                 if (stream && top && !exp_group_.empty() &&
-                    (exp_group_.size() == kGroupMax || exp_base_ + exp_group_.size() != before))
+                    ((M_ - before) % kGroupMax == 0 || exp_base_ + exp_group_.size() != before))
                     ZXA_TRY(flush_group());
                 if (stream && top)
                 {
@@ -1013,7 +1021,8 @@ int Sim::execute()
                     continue;
                 }
                 ZXA_TRY(flush_group());
-                ZXA_TRY(settle());
+                ZXA_TRY(settle(size_t(1) << (top ? before : active_bits())));
+                valid_ = std::max(valid_, size_t(1) << active_bits());
                 if (top)
                     ZXA_TRY(u3_expand_apply(ctx_, dstate_, prec_, active_bits(), eg));
                 else
@@ -1133,7 +1142,7 @@ int Sim::execute()
         ZXA_TRY(circuit_.run(ctx_, dstate_));
     ZXA_TRY(flush_pass());
     ZXA_TRY(flush_group());
-    ZXA_TRY(settle());
+    ZXA_TRY(settle(size_t(1) << M_));
     ZXA_HIP(hipStreamSynchronize(ctx_.stream));
     executed_ = true;
     return OK;
