@@ -167,3 +167,47 @@ def test_batches(gpu_engine, prec, widths, seg):
             assert abs(norms[k] - 1.0) < TOL[prec]
             assert np.max(np.abs(grads[k] - want[k][1])) < 12 * tol
     b.close()
+
+
+def layered(n, kind, layers, seed):
+    from zxh_adae_amd import workloads as W
+    rng = np.random.default_rng(seed)
+    gates = []
+    for _ in range(layers):
+        qs = range(n) if kind != "part" else [q for q in range(n) if rng.random() < 0.8]
+        gates += [(W.U3, 0, q, *rng.uniform(0, 6, 3)) for q in qs]
+        if kind == "flipped":
+            gates += [(W.X, 0, int(q), 0, 0, 0) for q in rng.choice(n, n // 2, replace=False)]
+        gates += [(W.CP, q, q + 1, float(rng.uniform(0, 6)), 0, 0) for q in range(n - 1)]
+        gates += [(W.P, 0, q, float(rng.uniform(0, 6)), 0, 0) for q in range(n)]
+    return gates
+
+
+@pytest.mark.parametrize("kind", ["whole", "part", "flipped"])
+@pytest.mark.parametrize("plain", [True, False])
+@pytest.mark.parametrize("prec,n", [("c128", 12), ("c128", 13), ("c128", 17), ("c128", 21), ("c64", 13), ("c64", 14),
+                                    ("c64", 18), ("c64", 22)])
+def test_engine_layers(gpu_engine, prec, n, plain, kind):
+    """The engine's batches behind a window (flipped: after X gates, whose
+    affine bit swaps the sides of a gate's pair), in tile passes; one and two
+    passes a layer, all targets below the tile and some left to a second."""
+    import oracle_py as O
+    from zxh_adae_amd import autotune as A
+    layers = 3
+    gates = layered(n, kind, layers, n)
+    o = O.OracleSim(n, False, plain)
+    o.gates(gates)
+    o.execute()
+    old = A.tune_get(f"circuit.bits.{prec}")
+    A.tune_set(f"circuit.bits.{prec}", 0)
+    try:
+        s = gpu_engine.ZXH(n, False, plain, precision=prec)
+        s.gates(gates)
+        s.set_timing(True)
+        s.execute()
+        launches = sum(s.timing(f)["launches"] for f in ("u3_tile", "fused"))
+        assert np.max(np.abs(s.get_state_array() - o.get_state())) < (1e-12 if prec == "c128" else 5e-6)
+    finally:
+        A.tune_set(f"circuit.bits.{prec}", old)
+    if plain and kind == "whole" and n in (17, 18):
+        assert launches == layers + 1  # two a layer, the end of one with the start of the next

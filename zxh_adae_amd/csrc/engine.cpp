@@ -577,6 +577,9 @@ int Sim::emit_u3(std::vector<U3Gate> &descs)
         return u3_apply(ctx_, dstate_, prec_, active_bits(), descs.data(), descs.size());
     }
     ZXA_TRY(flush_wide());
+    ZXA_TRY(turn(descs));
+    if (descs.empty())
+        return OK;
     const unsigned low = tile_low_bits(prec_);
     const unsigned n = active_bits();
     // Complex128 (X and CX as affine updates): a gate whose target the
@@ -691,6 +694,106 @@ int Sim::emit_u3(std::vector<U3Gate> &descs)
             pass_high_++;
     }
     return OK;
+}
+
+// A batch of several passes behind the window of the pending pass: the gates
+// of the batch that share a tile with the pass's go into the same sweep, after
+// the window (turn_pass_apply), where the rest of the batch then takes a pass
+// fewer.  They leave descs, and nothing stays pending.  (25 qubits of
+// complex128, the second layer of a QAOA circuit: four sweeps of 200 to 240 us
+// were three, of 298, 215 and 207; its layers of U3 and CP gates 1.3 times as
+// fast, complex64 1.1 to 1.2 times.)
+int Sim::turn(std::vector<U3Gate> &descs)
+{
+    const unsigned n = active_bits();
+    if (pass_u3_.empty() || pass_diag_.empty() || pass_has_fan_ || valid_ == 0 || !exp_group_.empty() ||
+        descs.size() <= tile_upper_slots(prec_) || !window_is_polynomial(n, pass_diag_.data(), pass_diag_.size()))
+        return OK;
+    auto target = [](const U3Gate &g) { return unsigned(__builtin_ctzll(g.delta)); };
+    auto passes = [&](const std::vector<unsigned> &ts) {
+        const unsigned low = tile_low_bits(prec_), slots = tile_upper_slots(prec_);
+        const size_t high = size_t(std::count_if(ts.begin(), ts.end(), [&](unsigned t) { return t >= low; }));
+        std::vector<std::vector<unsigned>> plan;
+        if (high <= slots)
+            return size_t(ts.empty() ? 0 : 1);
+        if (tune_get(prec_ == C64 ? "tile.wide.c64" : "tile.wide.c128") == 1 &&
+            tile_layer_plan(prec_, n, -1, ts, plan))
+            return plan.size();
+        return (high + slots - 1) / slots;
+    };
+    std::vector<unsigned> all;
+    for (const U3Gate &g : descs)
+        all.push_back(target(g));
+    // the tile geometry that leaves the fewest passes, the longest runs among
+    // equals
+    size_t least = passes(all);
+    int geometry = -1;
+    uint64_t joins = 0;
+    for (int seg = 6; seg >= 3; seg--)
+    {
+        const unsigned low = tile_low_bits(prec_, seg), slots = tile_upper_slots(prec_, seg);
+        uint64_t tile = 0;
+        for (const U3Gate &g : pass_u3_)
+            tile |= target(g) >= low ? g.delta : 0;
+        if (unsigned(__builtin_popcountll(tile)) > slots)
+            continue;
+        uint64_t take = 0, left = 0;
+        for (unsigned t : all)
+        {
+            const uint64_t bit = uint64_t(1) << t;
+            if (t < low)
+                continue;
+            if (!(tile & bit) && unsigned(__builtin_popcountll(tile)) == slots)
+            {
+                left |= bit;
+                continue;
+            }
+            // (targets outside the pass's tile take what slots are free)
+            tile |= bit;
+            take |= bit;
+        }
+        std::vector<unsigned> rest;
+        for (unsigned t : all)
+        {
+            // low targets fit any pass: they ride here when nothing else is left
+            if (t < low && left == 0)
+                take |= uint64_t(1) << t;
+            if (!((take >> t) & 1u))
+                rest.push_back(t);
+        }
+        const size_t k = passes(rest);
+        if (k < least)
+        {
+            least = k;
+            geometry = seg;
+            joins = take;
+        }
+    }
+    if (geometry < 0)
+        return OK;
+    std::vector<U3Gate> second, rest;
+    for (const U3Gate &g0 : descs)
+    {
+        U3Gate g = g0;
+        if (g.packed_sel >> 63)
+        {
+            // beta = 1: the even side is the target-bit-one element
+            const double sw[8] = {g0.u[6], g0.u[7], g0.u[4], g0.u[5], g0.u[2], g0.u[3], g0.u[0], g0.u[1]};
+            std::memcpy(g.u, sw, sizeof(sw));
+            g.packed_sel = g.delta;
+        }
+        (((joins & g.delta) != 0) ? second : rest).push_back(g);
+    }
+    descs.swap(rest);
+    ZXA_TRY(settle());
+    const int rc = turn_pass_apply(ctx_, dstate_, prec_, n, pass_u3_.data(), pass_u3_.size(), pass_diag_.data(),
+                                   pass_diag_.size(), second.data(), second.size(), geometry);
+    pass_u3_.clear();
+    pass_fan_.clear();
+    pass_diag_.clear();
+    pass_support_ = 0;
+    pass_high_ = 0;
+    return rc;
 }
 
 void Sim::Acc::merge()

@@ -150,6 +150,7 @@ class Sim
     int flush_diag(std::vector<DiagGate> &window);
     int flush_u3(std::vector<Acc> &pend, size_t &count);
     int emit_u3(std::vector<U3Gate> &descs);
+    int turn(std::vector<U3Gate> &descs);
     int flush_pass();
     bool fusable() const;
     int resize_reset(size_t M);
