@@ -866,8 +866,8 @@ int Sim::flush_u3(std::vector<Acc> &pend, size_t &count)
 // times).  Above it where it has more than a layer or so: its tables and plan
 // are paid once, and one layer of a resident state is a pass or two either
 // way (complex128, 20 bits: one layer 60 us in tile passes and 74 here, two
-// 128 and 93, ten 535 and 323; 21 bits 71 and 103, 141 and 151, 600 and 556.
-// complex64, 21 bits: 67 and 85, 129 and 110, 546 and 412; 22 bits 664 and 755
+// 106 and 93, ten 399 and 323; 21 bits 69 and 103, 124 and 151, 544 and 556.
+// complex64, 21 bits: 67 and 85, 112 and 110, 432 and 412; 22 bits 608 and 755
 // for ten).  A state that grows gate by gate costs a launch per new bit
 // besides: one layer of 18 bits 125 and 111, of 20 complex64 122 and 141.
 bool Sim::suits_lds() const
