@@ -210,6 +210,15 @@ int zxh_window_table(size_t nbits, const uint64_t *sel0, const uint64_t *sel1, c
  * this way.  Host only; needs no device.  No reference counterpart. */
 int zxh_tile_layer_plan(int precision, size_t nbits, int geometry, const uint32_t *targets, size_t ntargets,
                         uint32_t *pass_of, size_t *npasses);
+/* How a circuit on a state of nbits address bits (at most 22 complex128, 23
+ * complex64) is split into the passes that execute it out of LDS: nops
+ * operations, kind[i] 0 a U3 (pair offset delta[i], selector sel0[i]), 1 a U3
+ * on the pairs whose even-side element sel1[i] selects, 2 a diagonal gate
+ * (sel0[i], sel1[i], ~0 as in zxh_k_diag); order[k] is the operation applied
+ * k-th and pass_of[k] its pass.  Host only; needs no device.  No reference
+ * counterpart. */
+int zxh_circuit_plan(int precision, size_t nbits, const uint32_t *kind, const uint64_t *delta, const uint64_t *sel0,
+                     const uint64_t *sel1, size_t nops, uint32_t *order, uint32_t *pass_of);
 /* diag_pending_push_p / try_push_cp / flush (kernels.h:36-41) as one call:
  * ngates entries, sel1[i] == ~0 marks a P gate (Z/Rz already lowered to P). */
 int zxh_k_diag(void *state, int precision, size_t local_bits, const uint64_t *sel0, const uint64_t *sel1,

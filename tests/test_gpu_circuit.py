@@ -49,6 +49,28 @@ def test_soups(gpu_engine, n, mode, prec):
     check(gpu_engine, n, W.random_mixed(n, 40 + 20 * n, 700 + n), prec, mode, (None, 0) if n > 11 else (None,))
 
 
+@pytest.mark.parametrize("prec", ["c128", "c64"])
+@pytest.mark.parametrize("kind", ["z", "rz", "p", "cp", "cx_cp", "unset"])
+@pytest.mark.parametrize("n", [1, 2, 3, 5])
+def test_no_superposition(gpu_engine, n, kind, prec):
+    """Default mode without U3 or H: a state of no address bits, whose phase
+    gates on set qubits have constant selectors."""
+    a, b = 0, n - 1
+    if n == 1 and kind in ("cp", "cx_cp"):
+        pytest.skip("needs two qubits")
+    gates = {"z": [(W.X, 0, b, 0, 0, 0), (W.Z, 0, b, 0, 0, 0)],
+             "rz": [(W.X, 0, b, 0, 0, 0), (W.RZ, 0, b, 0.3, 0, 0)],
+             "p": [(W.X, 0, b, 0, 0, 0), (W.P, 0, b, 0.3, 0, 0), (W.X, 0, b, 0, 0, 0), (W.P, 0, b, 0.5, 0, 0)],
+             "cp": [(W.X, 0, a, 0, 0, 0), (W.X, 0, b, 0, 0, 0), (W.CP, a, b, 0.3, 0, 0)],
+             "cx_cp": [(W.X, 0, a, 0, 0, 0), (W.CX, a, b, 0, 0, 0), (W.CP, a, b, 0.3, 0, 0)],
+             "unset": [(W.P, 0, b, 0.3, 0, 0)]}[kind]
+    s = check(gpu_engine, n, gates, prec, "lazy", (None, 0))
+    s.set_seed(5)
+    s.measure(7)
+    at = np.flatnonzero(s.get_state_array())
+    assert at.size == 1 and np.all(s.results_bits() == [(at[0] >> (n - 1 - q)) & 1 for q in range(n)])
+
+
 @pytest.mark.parametrize("prec,n", [("c128", 13), ("c64", 14), ("c128", 14), ("c64", 15), ("c128", 17)])
 def test_no_gates_and_one_gate(gpu_engine, prec, n):
     s = check(gpu_engine, n, [], prec, "plain")

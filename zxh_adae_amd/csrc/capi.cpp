@@ -511,6 +511,35 @@ int zxh_tile_layer_plan(int precision, size_t nbits, int geometry, const uint32_
     return ZXH_OK;
 }
 
+int zxh_circuit_plan(int precision, size_t nbits, const uint32_t *kind, const uint64_t *delta, const uint64_t *sel0,
+                     const uint64_t *sel1, size_t nops, uint32_t *order, uint32_t *pass_of)
+{
+    if (nops && (!kind || !delta || !sel0 || !sel1 || !order || !pass_of))
+        return fail(ZXH_EINVAL, "null argument");
+    if (precision != ZXH_C128 && precision != ZXH_C64)
+        return fail(ZXH_EINVAL, "precision must be ZXH_C128 or ZXH_C64");
+    if (nbits > zxa::lds_tile_bits(precision) + zxa::kLdsOuter)
+        return fail(ZXH_EINVAL, "circuit plan: state too wide");
+    zxa::LdsCircuit c;
+    c.begin(unsigned(nbits), precision);
+    for (size_t i = 0; i < nops; i++)
+    {
+        int rc;
+        if (kind[i] == 2)
+        {
+            const zxa::DiagGate d = {sel0[i], sel1[i], 0.0};
+            rc = c.window(&d, 1);
+        }
+        else if (kind[i] < 2)
+            rc = c.swap(delta[i], sel0[i], kind[i] ? &sel1[i] : nullptr);
+        else
+            rc = fail(ZXH_EINVAL, "circuit plan: unknown kind of operation");
+        if (rc)
+            return rc;
+    }
+    return c.schedule(order, pass_of);
+}
+
 int zxh_k_diag(void *state, int precision, size_t local_bits, const uint64_t *sel0, const uint64_t *sel1,
                const double *theta, size_t ngates)
 {

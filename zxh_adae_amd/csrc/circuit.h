@@ -83,6 +83,9 @@ class LdsCircuit
     // Runs the operations on the state (2^bits amplitudes), from |0...0>,
     // which need not have been written.
     int run(Ctx &ctx, void *state);
+    // The plan alone, on the host: the operations in the order they are
+    // applied, and the pass of each.
+    int schedule(uint32_t *order, uint32_t *pass_of);
 
   private:
     struct Op
@@ -103,6 +106,8 @@ class LdsCircuit
     // A planned pass: its kernel arguments and where its tables are.
     struct Pass;
     int push(const U3Gate &g, const uint64_t *ctrl);
+    void start();
+    int next_pass();
     void plan();
     void place();
     int stage(Ctx &ctx, bool fresh, Pass &out);

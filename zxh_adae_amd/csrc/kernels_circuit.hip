@@ -676,7 +676,10 @@ void LdsCircuit::plan()
     for (; at < rest_.size(); at++)
     {
         if (at >= kMaxScan || drafts_.size() + 4 > kMaxSteps || diags + pending_.size() >= kMaxDiags ||
-            dgates_.size() + ddiags_.size() > kMaxDeferred || (simple_ && ddelta == all))
+            dgates_.size() + ddiags_.size() > kMaxDeferred ||
+            // every address bit has a deferred gate (a state of no address
+            // bits, whose phase gates have constant selectors, has neither)
+            (simple_ && ddelta != 0 && ddelta == all))
             break;
         const Op &o = ops_[rest_[at]];
         if (o.kind == 2u)
@@ -1017,11 +1020,44 @@ int LdsCircuit::launch(Ctx &ctx, void *state, const std::vector<Pass> &passes)
     return ctx.ring.done(ctx.stream);
 }
 
-int LdsCircuit::run(Ctx &ctx, void *state)
+void LdsCircuit::start()
 {
     rest_.resize(ops_.size());
     for (size_t i = 0; i < ops_.size(); i++)
         rest_[i] = uint32_t(i);
+}
+
+int LdsCircuit::next_pass()
+{
+    const size_t before = rest_.size();
+    plan();
+    if (rest_.size() == before && before)
+    {
+        set_error("circuit: no operation fits a pass");
+        return ESTATE;
+    }
+    return OK;
+}
+
+int LdsCircuit::schedule(uint32_t *order, uint32_t *pass_of)
+{
+    size_t at = 0;
+    uint32_t pass = 0;
+    for (start(); !rest_.empty(); pass++)
+    {
+        ZXA_TRY(next_pass());
+        for (uint32_t o : order_)
+        {
+            order[at] = o;
+            pass_of[at++] = pass;
+        }
+    }
+    return OK;
+}
+
+int LdsCircuit::run(Ctx &ctx, void *state)
+{
+    start();
     // the first pass by itself, then three and up to eight with one table
     // copy and one table launch: the device works on one lot while the host
     // plans the next
@@ -1043,13 +1079,7 @@ int LdsCircuit::run(Ctx &ctx, void *state)
         size_t tabs = 0;
         while ((fresh || !rest_.empty()) && passes.size() < lot && tabs < kTabBytes)
         {
-            const size_t before = rest_.size();
-            plan();
-            if (rest_.size() == before && before)
-            {
-                set_error("circuit: no operation fits a pass");
-                return ESTATE;
-            }
+            ZXA_TRY(next_pass());
             passes.emplace_back();
             ZXA_TRY(stage(ctx, fresh, passes.back()));
             tabs += (size_t(passes.back().P.nwin) << passes.back().P.bits) * elem_bytes(prec_);
