@@ -3,6 +3,8 @@
 reference applies one sweep per gate, zxh.cpp:390-428), so the checks are its
 contract: every operation once, operations that do not commute in the
 circuit's order, a pass's pair offsets within one tile."""
+import time
+
 import numpy as np
 import pytest
 
@@ -109,6 +111,29 @@ def test_no_address_bits(prec, ops):
 def test_random_circuits(prec, nbits, kinds):
     rng = np.random.default_rng(nbits)
     check_plan(prec, nbits, random_ops(rng, nbits, 150, kinds))
+
+
+def plan_seconds(nbits, nops):
+    """Gates whose offsets take two random bits, on the host clock."""
+    rng = np.random.default_rng(1)
+    b = rng.integers(nbits, size=nops)
+    sel = np.uint64(1) << b.astype(np.uint64)
+    delta = sel | np.uint64(1) << ((b + 1 + rng.integers(nbits - 1, size=nops)) % nbits).astype(np.uint64)
+    kind, zero = np.zeros(nops, np.uint32), np.zeros(nops, np.uint64)
+    order, pass_of = np.empty(nops, np.uint32), np.empty(nops, np.uint32)
+    t = time.perf_counter()
+    check(_lib.load().zxh_circuit_plan(_lib.ZXH_C128, nbits, kind.ctypes.data, delta.ctypes.data, sel.ctypes.data,
+                                       zero.ctypes.data, nops, order.ctypes.data, pass_of.ctypes.data))
+    return time.perf_counter() - t
+
+
+def test_time_grows_with_the_length():
+    """Sixteen times the operations: 16 times the time when a pass touches
+    only the operations it looks at, 195 times when it moved all that follow.
+    The bound is three times the first, the least of three runs each."""
+    small = min(plan_seconds(16, 50_000) for _ in range(3))
+    large = min(plan_seconds(16, 800_000) for _ in range(3))
+    assert large < 48 * small, (small, large)
 
 
 def test_bad_arguments():

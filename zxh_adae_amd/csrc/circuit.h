@@ -118,7 +118,13 @@ class LdsCircuit
     std::vector<Op> ops_;
     std::vector<std::array<double, 8>> mats_;
     // planning of a pass
-    std::vector<uint32_t> rest_, later_;          // operations not yet in a pass
+    std::vector<uint32_t> rest_;                  // from head_ on: operations not yet in a pass
+    std::vector<uint32_t> later_;                 // of those, looked at for a pass and deferred
+    size_t head_ = 0;
+    bool left() const
+    {
+        return head_ < rest_.size();
+    }
     std::vector<uint32_t> order_;                 // operations of the pass, by draft
     std::vector<Draft> drafts_;
     std::vector<uint32_t> vec_, piv_, red_, mix_; // the tile's offsets; elimination
