@@ -1389,6 +1389,9 @@ int Sim::get_state(double *out, size_t out_len)
         set_error("output buffer too small");
         return EINVAL_;
     }
+    // what a caller's default stream still writes to the state (device_ptr) is
+    // seen: the simulator's own stream does not wait for it
+    ZXA_HIP(hipStreamSynchronize(nullptr));
     return virtual_state(ctx_, dstate_, prec_, unsigned(N_), unsigned(m_), rows_.data(), b_.data(), gphase_.real(),
                          gphase_.imag(), out);
 }
