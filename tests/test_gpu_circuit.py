@@ -71,6 +71,25 @@ def test_no_superposition(gpu_engine, n, kind, prec):
     assert at.size == 1 and np.all(s.results_bits() == [(at[0] >> (n - 1 - q)) & 1 for q in range(n)])
 
 
+@pytest.mark.parametrize("prec", ["c128", "c64"])
+@pytest.mark.parametrize("n,gates", [(2, [(W.X, 0, 1, 0, 0, 0), (W.P, 0, 1, 0.3, 0, 0)]), (3, W.hadamard_all(3))])
+def test_knob_at_zero_is_never(gpu_engine, n, gates, prec):
+    """Also for a state of no address bits."""
+    name = f"circuit.bits.{prec}"
+    old = A.tune_get(name)
+    s = gpu_engine.ZXH(n, False, False, precision=prec)
+    s.gates(gates)
+    s.set_timing(True)
+    try:
+        for knob, launches in ((0, 0), (old, 1)):
+            A.tune_set(name, knob)
+            s.reset_timing()
+            s.execute()
+            assert s.timing("fused")["launches"] == launches
+    finally:
+        A.tune_set(name, old)
+
+
 @pytest.mark.parametrize("prec,n", [("c128", 13), ("c64", 14), ("c128", 14), ("c64", 15), ("c128", 17)])
 def test_no_gates_and_one_gate(gpu_engine, prec, n):
     s = check(gpu_engine, n, [], prec, "plain")

@@ -872,7 +872,8 @@ int Sim::flush_u3(std::vector<Acc> &pend, size_t &count)
 // besides: one layer of 18 bits 125 and 111, of 20 complex64 122 and 141.
 bool Sim::suits_lds() const
 {
-    if (M_ > size_t(tune_get(prec_ == C64 ? "circuit.bits.c64" : "circuit.bits.c128")))
+    const size_t widest = size_t(tune_get(prec_ == C64 ? "circuit.bits.c64" : "circuit.bits.c128"));
+    if (widest == 0 || M_ > widest)
         return false;
     if (M_ < tile_min_bits(prec_) || (!eager_ && M_ <= 18))
         return true;
