@@ -127,6 +127,28 @@ def test_a_window_larger_than_a_pass_takes(gpu_engine):
 
 
 @pytest.mark.parametrize("prec", ["c128", "c64"])
+@pytest.mark.parametrize("mode", ["plain", "lazy"])
+@pytest.mark.parametrize("n,count", [(1, 65), (2, 200), (5, 64), (7, 128), (13, 129), (14, 300), (15, 1000), (18, 300)])
+def test_windows_of_equal_gates(gpu_engine, n, count, mode, prec):
+    """Windows above 64 gates, whose equal ones become one: P and CP gates on
+    random qubits in both orders, with X gates between them (selectors of
+    either sign) and, in the last window, after CX transport.  Angles to 0.01:
+    see the test above."""
+    r = W.SplitMix64(1000 * n + count)
+    gates = W.hadamard_all(n)
+    for part in range(3):
+        if part == 2 and n > 1:
+            gates += [(W.CX, q, (q + 1) % n, 0, 0, 0) for q in range(n)]
+        for k in range(count):
+            a, b = r.below(n), r.below(n)
+            if k % 7 == 3:
+                gates.append((W.X, 0, a, 0, 0, 0))
+            gates.append((W.P, 0, a, 0.01 * r.uniform(), 0, 0) if a == b else (W.CP, a, b, 0.01 * r.uniform(), 0, 0))
+        gates += [(W.U3, 0, q, r.uniform() * 6, r.uniform() * 6, r.uniform() * 6) for q in range(n)]
+    check(gpu_engine, n, gates, prec, mode, (None, 0))
+
+
+@pytest.mark.parametrize("prec", ["c128", "c64"])
 @pytest.mark.parametrize("n,layers", [(14, 20), (17, 9), (20, 6), (21, 3), (22, 2)])
 def test_layers_over_tiles(gpu_engine, n, layers, prec):
     """Layers with CP ladders: passes that carry parts of several layers, up

@@ -117,6 +117,7 @@ class LdsCircuit
     bool simple_ = true; // every gate on one address bit, its selector that bit
     std::vector<Op> ops_;
     std::vector<std::array<double, 8>> mats_;
+    std::vector<uint32_t> seen_; // a window's hash table: 0, or one past an operation
     // planning of a pass
     std::vector<uint32_t> rest_;                  // from head_ on: operations not yet in a pass
     std::vector<uint32_t> later_;                 // of those, looked at for a pass and deferred

@@ -179,6 +179,10 @@ struct WinTask
     uint64_t win; // const LdsWin *
 };
 constexpr int kFactors = 64;
+// Gates of a table's sum, read together into LDS (one by one from memory, each
+// waiting for the one before, a gate took 0.25 us).
+constexpr int kTabGates = 128;
+static_assert(sizeof(LdsDiag) == 32 && 2 * kTabGates == 256, "two 16-byte loads a gate, one per thread");
 
 template <bool kC64>
 __global__ __launch_bounds__(256) void window_kernel(const WinTask *__restrict__ tasks, uint32_t bits,
@@ -187,23 +191,33 @@ __global__ __launch_bounds__(256) void window_kernel(const WinTask *__restrict__
                                                      double2 *__restrict__ factors)
 {
     __shared__ LdsWin W;
+    __shared__ LdsDiag sh[kTabGates];
     const WinTask task = tasks[blockIdx.y];
     if (blockIdx.x < tblocks)
     {
         const uint32_t x = blockIdx.x * blockDim.x + threadIdx.x;
-        if (x >> bits)
-            return;
-        const LdsDiag *gates = reinterpret_cast<const LdsDiag *>(task.gates);
         const uint32_t count = uint32_t(task.count);
         // the angles' sum with its rounding errors carried beside it
         double th = 0.0, lo = 0.0;
-        for (uint32_t g = 0; g < count; g++)
+        for (uint32_t g0 = 0; g0 < count; g0 += kTabGates)
         {
-            const double a = (odd(gates[g].s0, x) & odd(gates[g].s1, x)) ? gates[g].theta : 0.0;
-            const double t = th + a, b = t - th;
-            lo += (th - (t - b)) + (a - b);
-            th = t;
+            const uint32_t n = min(uint32_t(kTabGates), count - g0);
+            const float4 *src = reinterpret_cast<const float4 *>(task.gates) + 2 * g0;
+            __syncthreads();
+            if (threadIdx.x < 2 * n)
+                reinterpret_cast<float4 *>(sh)[threadIdx.x] = src[threadIdx.x];
+            __syncthreads();
+#pragma unroll 4
+            for (uint32_t g = 0; g < n; g++)
+            {
+                const double a = (odd(sh[g].s0, x) & odd(sh[g].s1, x)) ? sh[g].theta : 0.0;
+                const double t = th + a, b = t - th;
+                lo += (th - (t - b)) + (a - b);
+                th = t;
+            }
         }
+        if (x >> bits)
+            return;
         double s, c;
         sincos(th + lo, &s, &c);
         typename CGeo<kC64>::T r;
@@ -491,6 +505,7 @@ constexpr size_t kTabBytes = size_t(32) << 20;   // window tables of one pass
 constexpr size_t kMaxLot = 8;                    // passes planned and staged together
 constexpr size_t kMaxSteps = 512;                // of one pass (128 KiB of its slot)
 constexpr size_t kMaxDiags = 2560;               // 80 KiB
+constexpr size_t kMergeFrom = 64;                // gates of a window above which equal ones are looked for
 constexpr size_t kMaxScan = 8192;                // operations looked at for one pass
 constexpr size_t kMaxDeferred = 192;             // of them deferred, where each is compared
 
@@ -560,8 +575,21 @@ int LdsCircuit::swap(uint64_t delta, uint64_t sel, const uint64_t *ctrl)
     return push(g, ctrl);
 }
 
+// Of a long window, gates with the same selectors become one, its angle their
+// sum with the rounding errors carried: a table takes time by the gate (3000
+// CP gates on 20 qubits, 190 of them different, took 0.8 ms).
 int LdsCircuit::window(const DiagGate *gates, size_t ngates)
 {
+    const bool merge = ngates > kMergeFrom;
+    const size_t first = ops_.size();
+    unsigned shift = 64;
+    std::vector<double> low;
+    if (merge)
+    {
+        while ((size_t(1) << (64 - shift)) < 2 * ngates)
+            shift--;
+        seen_.assign(size_t(1) << (64 - shift), 0u);
+    }
     for (size_t i = 0; i < ngates; i++)
     {
         const DiagGate &d = gates[i];
@@ -570,8 +598,30 @@ int LdsCircuit::window(const DiagGate *gates, size_t ngates)
             set_error("circuit: diagonal selector outside the state");
             return EINVAL_;
         }
-        ops_.push_back({2u, 0u, pack32(d.s0), d.s1 == kNoSel ? kTrue : pack32(d.s1), d.theta, 0u});
+        Op o = {2u, 0u, pack32(d.s0), d.s1 == kNoSel ? kTrue : pack32(d.s1), d.theta, 0u};
+        if (merge)
+        {
+            if (o.s1 != kTrue && o.s0 > o.s1)
+                std::swap(o.s0, o.s1);
+            uint64_t h = ((uint64_t(o.s0) << 32 | o.s1) * 0x9e3779b97f4a7c15ull) >> shift;
+            for (; seen_[h] != 0; h = (h + 1) & (seen_.size() - 1))
+                if (ops_[seen_[h] - 1].s0 == o.s0 && ops_[seen_[h] - 1].s1 == o.s1)
+                    break;
+            if (seen_[h] != 0)
+            {
+                double &th = ops_[seen_[h] - 1].theta;
+                const double t = th + o.theta, b = t - th;
+                low[seen_[h] - 1 - first] += (th - (t - b)) + (o.theta - b);
+                th = t;
+                continue;
+            }
+            seen_[h] = uint32_t(ops_.size() + 1);
+            low.push_back(0.0);
+        }
+        ops_.push_back(o);
     }
+    for (size_t i = 0; i < low.size(); i++)
+        ops_[first + i].theta = turn(ops_[first + i].theta) + low[i];
     return OK;
 }
 
@@ -889,17 +939,22 @@ int LdsCircuit::stage(Ctx &ctx, bool fresh, Pass &out)
         }
         const uint32_t g0 = uint32_t(diags.size());
         win.clear();
+        for (uint32_t j = 0; j < d.count && tile; j++)
+        {
+            const Op &o = ops_[order_[d.first + j]];
+            win.push_back({uint64_t(o.s0 & kAlpha32) | (uint64_t(o.s0 >> 31) << 63),
+                           o.s1 == kTrue ? kNoSel : uint64_t(o.s1 & kAlpha32) | (uint64_t(o.s1 >> 31) << 63),
+                           o.theta});
+        }
+        const bool table = !tile || (units && window_is_polynomial(bits_, win.data(), win.size()));
         for (uint32_t j = 0; j < d.count; j++)
         {
             const Op &o = ops_[order_[d.first + j]];
-            diags.push_back({form(o.s0), form(o.s1), tile ? o.s0 & kAlpha32 : 0u, tile ? o.s1 & kAlpha32 : 0u,
-                             turn(o.theta), 0.0});
-            if (tile)
-                win.push_back({uint64_t(o.s0 & kAlpha32) | (uint64_t(o.s0 >> 31) << 63),
-                               o.s1 == kTrue ? kNoSel : uint64_t(o.s1 & kAlpha32) | (uint64_t(o.s1 >> 31) << 63),
-                               o.theta});
+            const uint32_t s0 = form(o.s0), s1 = form(o.s1);
+            if (!table || (s0 != 0 && s1 != 0)) // (a table's gate that needs a bit outside the tile holds nowhere in it)
+                diags.push_back({s0, s1, tile ? o.s0 & kAlpha32 : 0u, tile ? o.s1 & kAlpha32 : 0u, turn(o.theta), 0.0});
         }
-        if (tile && !(units && window_is_polynomial(bits_, win.data(), win.size())))
+        if (!table)
         {
             st.kind = 3u;
             st.slot[0] = g0;
