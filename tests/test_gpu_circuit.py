@@ -159,6 +159,28 @@ def test_layers_over_tiles(gpu_engine, n, layers, prec):
     check(gpu_engine, n, W.random_layers(n, layers, 50 + n), prec, "plain", (top, 0))
 
 
+@pytest.mark.parametrize("prec,n", [("c128", 14), ("c128", 18), ("c128", 19), ("c64", 15), ("c64", 20), ("c64", 21)])
+@pytest.mark.parametrize("mode", ["plain", "lazy"])
+def test_windows_of_both_kinds(gpu_engine, n, mode, prec):
+    """Windows that split by tile and coordinate and windows that do not, in
+    one pass and in turn, at both ends of the states whose tables hold every
+    tile, and one bit above."""
+    r = W.SplitMix64(31 * n)
+    gates = W.hadamard_all(n)
+    for layer in range(4):
+        if layer % 2:
+            gates += [(W.CX, q, (q + 3) % n, 0, 0, 0) for q in range(n)]
+        for k in range(2 * n):
+            a, b = r.below(n), r.below(n - 1)
+            gates.append((W.CP, a, b + (b >= a), r.uniform(), 0, 0))
+        if layer % 2:
+            gates += [(W.CX, q, (q + 3) % n, 0, 0, 0) for q in reversed(range(n))]
+        gates += [(W.U3, 0, q, r.uniform() * 6, r.uniform() * 6, r.uniform() * 6) for q in range(0, n, 1 + layer % 2)]
+        gates += [(W.CP, q, q + 1, r.uniform(), 0, 0) for q in range(n - 1)]
+        gates += [(W.H, 0, q, 0, 0, 0) for q in range(3)]
+    check(gpu_engine, n, gates, prec, mode, (None, 0))
+
+
 @pytest.mark.parametrize("prec", ["c128", "c64"])
 @pytest.mark.parametrize("n", [14, 17, 20])
 @pytest.mark.parametrize("kind", ["chain", "reverse", "soup", "windows", "qft"])

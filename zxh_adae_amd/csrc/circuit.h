@@ -27,6 +27,19 @@ constexpr unsigned lds_tile_bits(int prec)
 {
     return prec == C64 ? 13u : 12u;
 }
+// Widest state whose windows that do not split by tile and coordinate (after
+// CX transport) are tabulated over all amplitudes, by every compute unit before
+// the pass, rather than summed gate by gate in the tiles, by as many as there
+// are tiles.  Four layers with 100 transported CP gates each, in us, gate by
+// gate and tabulated (and in tile passes): complex128, 14 bits 339, 200 (295),
+// 18 bits 391, 294 (351); complex64, 16 bits 575, 250 (358), 20 bits 658, 503
+// (600).  A table of 2^20 complex128 or 2^21 complex64 amplitudes, 16 MiB each,
+// takes the whole chip as long as the tiles take, which have a compute unit
+// each there (0.6 and 0.44 us a gate).
+constexpr unsigned lds_table_bits(int prec)
+{
+    return prec == C64 ? 20u : 18u;
+}
 constexpr int kLdsOuter = 10;  // most address bits outside a tile
 constexpr int kLdsWindows = 8; // most windows of a pass over tiles
 

@@ -172,12 +172,17 @@ __device__ __forceinline__ void gates_step(typename CGeo<kC64>::T *amp, const St
 // state of several tiles): per window and tile 64 factors of exp(i (C + sum_i
 // c_i l_i)), by groups of coordinate bits, 32 for bits 0-4 (with C), 16 for
 // bits 5-8 and 16 for bits 9-12.
+// A window whose selectors do not split so has a table of every tile, formed
+// by a launch of its own over tile index and coordinates together (bits: the
+// state's), and factors of 1.
 struct WinTask
 {
     uint64_t gates; // const LdsDiag *
     uint64_t count;
-    uint64_t win; // const LdsWin *
+    uint64_t win;   // const LdsWin *
+    uint64_t out;   // the table's first entry; kNoTable: formed by the other launch
 };
+constexpr uint64_t kNoTable = ~uint64_t(0);
 constexpr int kFactors = 64;
 // Gates of a table's sum, read together into LDS (one by one from memory, each
 // waiting for the one before, a gate took 0.25 us).
@@ -195,6 +200,8 @@ __global__ __launch_bounds__(256) void window_kernel(const WinTask *__restrict__
     const WinTask task = tasks[blockIdx.y];
     if (blockIdx.x < tblocks)
     {
+        if (task.out == kNoTable)
+            return;
         const uint32_t x = blockIdx.x * blockDim.x + threadIdx.x;
         const uint32_t count = uint32_t(task.count);
         // the angles' sum with its rounding errors carried beside it
@@ -223,7 +230,7 @@ __global__ __launch_bounds__(256) void window_kernel(const WinTask *__restrict__
         typename CGeo<kC64>::T r;
         r.x = c;
         r.y = s;
-        out[(uint64_t(blockIdx.y) << bits) + x] = r;
+        out[task.out + x] = r;
         return;
     }
     static_assert(sizeof(LdsWin) / sizeof(double) <= 256, "one load per thread");
@@ -287,6 +294,7 @@ struct CPass
     uint32_t bits, ntiles, outer;
     uint32_t nsteps, nwin;
     uint32_t fresh; // the state is |0...0>, not yet written
+    uint32_t wfull; // bit k: window k has a table per tile
 };
 
 // The circuit, or a pass of it.  A workgroup holds a tile in LDS from the
@@ -390,7 +398,16 @@ __global__ __launch_bounds__(kThreads) void circuit_kernel(typename CGeo<kC64>::
             // before it (past the last window those of the first amplitudes'
             // worth of any window, or of the state, unused)
             T pf[kPf];
-            const T *src = P.nwin ? tabs + (uint64_t(min(win, P.nwin - 1)) << P.bits) : state;
+            const T *src = state;
+            if (P.nwin)
+            {
+                const uint32_t wi = min(win, P.nwin - 1);
+                uint64_t table = wi;
+                if constexpr (kTile)
+                    table += uint64_t(__builtin_popcount(P.wfull & ((1u << wi) - 1))) * (P.ntiles - 1) +
+                             ((P.wfull >> wi) & 1u ? tile : 0u);
+                src = tabs + (table << P.bits);
+            }
 #pragma unroll
             for (int k = 0; k < kPf; k++)
                 pf[k] = src[kTile ? tid + k * nt : min(tid + k * nt, size - 1)];
@@ -415,7 +432,8 @@ __global__ __launch_bounds__(kThreads) void circuit_kernel(typename CGeo<kC64>::
                 else if constexpr (kTile)
                 {
                     // a window whose selectors do not split by tile and
-                    // coordinate: gate by gate
+                    // coordinate, of a state wider than lds_table_bits: gate by
+                    // gate
                     const uint32_t g0 = h.slot[0], g1 = h.slot[1];
                     double th[kPer] = {};
                     for (uint32_t g = g0; g < g1; g++)
@@ -844,7 +862,16 @@ struct LdsCircuit::Pass
 {
     CPass P;
     const char *steps, *diags, *wins;
-    std::vector<std::pair<uint32_t, uint32_t>> ranges; // per table: its diagonal gates
+    std::vector<std::pair<uint32_t, uint32_t>> ranges; // per window with a table: its diagonal gates
+    // tables of 2^P.bits entries that window k comes after
+    size_t tables(size_t k) const
+    {
+        return k + size_t(__builtin_popcount(P.wfull & ((1u << std::min<size_t>(k, 31)) - 1))) * (P.ntiles - 1);
+    }
+    size_t tables() const
+    {
+        return tables(ranges.size());
+    }
 };
 
 int LdsCircuit::stage(Ctx &ctx, bool fresh, Pass &out)
@@ -947,27 +974,38 @@ int LdsCircuit::stage(Ctx &ctx, bool fresh, Pass &out)
                            o.theta});
         }
         const bool table = !tile || (units && window_is_polynomial(bits_, win.data(), win.size()));
+        // (over the tile index and the coordinates, where a table has them all)
+        const bool full = !table && bits_ <= lds_table_bits(prec_);
+        auto index_form = [&](uint32_t sel) {
+            uint32_t t = 0;
+            for (size_t k = 0; k < outer.size() && full; k++)
+                t |= ((sel >> outer[k]) & 1u) << (w + k);
+            return t;
+        };
         for (uint32_t j = 0; j < d.count; j++)
         {
             const Op &o = ops_[order_[d.first + j]];
-            const uint32_t s0 = form(o.s0), s1 = form(o.s1);
+            const uint32_t s0 = form(o.s0) | index_form(o.s0), s1 = form(o.s1) | index_form(o.s1);
             if (!table || (s0 != 0 && s1 != 0)) // (a table's gate that needs a bit outside the tile holds nowhere in it)
                 diags.push_back({s0, s1, tile ? o.s0 & kAlpha32 : 0u, tile ? o.s1 & kAlpha32 : 0u, turn(o.theta), 0.0});
         }
-        if (!table)
+        if (!table && !full)
         {
             st.kind = 3u;
             st.slot[0] = g0;
             st.slot[1] = uint32_t(diags.size());
             continue;
         }
+        P.wfull |= uint32_t(full) << (tile ? out.ranges.size() : 0);
         out.ranges.push_back({g0, uint32_t(diags.size())});
         if (!tile)
             continue;
-        window_polynomial(bits_, win.data(), win.size(), poly);
         wins.emplace_back();
         LdsWin &W = wins.back();
         std::memset(&W, 0, sizeof(W));
+        if (full)
+            continue;
+        window_polynomial(bits_, win.data(), win.size(), poly);
         for (size_t k = 0; k < outer.size(); k++)
         {
             for (unsigned i = 0; i < w; i++)
@@ -1006,12 +1044,28 @@ int LdsCircuit::launch(Ctx &ctx, void *state, const std::vector<Pass> &passes)
     const bool c64 = prec_ == C64;
     const uint32_t w = passes[0].P.bits;
     const bool tile = w != bits_;
-    std::vector<WinTask> tasks;
+    // (a window with a table per tile twice: its factors, and its table)
+    std::vector<WinTask> tasks, wide;
+    size_t ntab = 0;
     for (const Pass &p : passes)
+    {
         for (size_t k = 0; k < p.ranges.size(); k++)
-            tasks.push_back({reinterpret_cast<uint64_t>(p.diags) + p.ranges[k].first * sizeof(LdsDiag),
-                             p.ranges[k].second - p.ranges[k].first,
-                             reinterpret_cast<uint64_t>(p.wins) + (tile ? k * sizeof(LdsWin) : 0)});
+        {
+            WinTask t = {reinterpret_cast<uint64_t>(p.diags) + p.ranges[k].first * sizeof(LdsDiag),
+                         p.ranges[k].second - p.ranges[k].first,
+                         reinterpret_cast<uint64_t>(p.wins) + (tile ? k * sizeof(LdsWin) : 0),
+                         uint64_t(ntab + p.tables(k)) << w};
+            if (tile && ((p.P.wfull >> k) & 1u))
+            {
+                wide.push_back(t);
+                t.out = kNoTable;
+            }
+            tasks.push_back(t);
+        }
+        ntab += p.tables();
+    }
+    const size_t nwin = tasks.size();
+    tasks.insert(tasks.end(), wide.begin(), wide.end());
     void *dr = nullptr;
     if (!tasks.empty())
         ZXA_TRY(ctx.ring.stage(tasks.data(), tasks.size() * sizeof(WinTask), ctx.stream, &dr));
@@ -1022,26 +1076,36 @@ int LdsCircuit::launch(Ctx &ctx, void *state, const std::vector<Pass> &passes)
     if (!tasks.empty())
     {
         const uint32_t outer = passes[0].P.outer;
-        const size_t tab_bytes = (tasks.size() << w) * elem_bytes(prec_);
-        auto need = [&](size_t windows) {
-            return (windows << w) * elem_bytes(prec_) + (tile ? (windows << outer) * kFactors * sizeof(double2) : 0);
+        auto need = [&](size_t tables, size_t windows) {
+            return (tables << w) * elem_bytes(prec_) + (tile ? (windows << outer) * kFactors * sizeof(double2) : 0);
         };
         // passes to come: the largest lot's at once (an allocation that grows
         // under way waits for the device, 1 ms of a first run in all)
-        ZXA_TRY(ctx.scratch_a.ensure(need(!left() ? tasks.size() : std::max(tasks.size(), kMaxLot * kLdsWindows))));
+        size_t bytes = need(ntab, nwin);
+        if (left())
+        {
+            const size_t most = kMaxLot * kLdsWindows;
+            bytes = std::max(bytes, need(most, most));
+            if (tile && !wide.empty())
+                bytes = std::max(bytes, need((kTabBytes >> w) / elem_bytes(prec_) + (size_t(kLdsWindows) << outer), most));
+        }
+        ZXA_TRY(ctx.scratch_a.ensure(bytes));
         tabs = static_cast<char *>(ctx.scratch_a.ptr);
-        factors = reinterpret_cast<double2 *>(tabs + tab_bytes);
-        const uint32_t tblocks = ((1u << w) + 255u) / 256u;
-        const uint32_t fblocks = tile ? ((1u << outer) + 3u) / 4u : 0u;
-        const dim3 grid(tblocks + fblocks, unsigned(tasks.size()));
+        factors = reinterpret_cast<double2 *>(tabs + (ntab << w) * elem_bytes(prec_));
         const WinTask *tk = static_cast<const WinTask *>(dr);
-        if (c64)
-            hipLaunchKernelGGL(window_kernel<true>, grid, dim3(256), 0, ctx.stream, tk, w, tblocks, outer,
-                               reinterpret_cast<float2 *>(tabs), factors);
-        else
-            hipLaunchKernelGGL(window_kernel<false>, grid, dim3(256), 0, ctx.stream, tk, w, tblocks, outer,
-                               reinterpret_cast<double2 *>(tabs), factors);
-        ZXA_HIP(hipGetLastError());
+        auto run = [&](uint32_t tblocks, uint32_t fblocks, size_t first, size_t count, uint32_t bits) {
+            const dim3 grid(tblocks + fblocks, unsigned(count));
+            if (c64)
+                hipLaunchKernelGGL(window_kernel<true>, grid, dim3(256), 0, ctx.stream, tk + first, bits, tblocks,
+                                   outer, reinterpret_cast<float2 *>(tabs), factors);
+            else
+                hipLaunchKernelGGL(window_kernel<false>, grid, dim3(256), 0, ctx.stream, tk + first, bits, tblocks,
+                                   outer, reinterpret_cast<double2 *>(tabs), factors);
+            return hip_check(hipGetLastError(), "window kernel launch");
+        };
+        ZXA_TRY(run(((1u << w) + 255u) / 256u, tile ? ((1u << outer) + 3u) / 4u : 0u, 0, nwin, w));
+        if (!wide.empty())
+            ZXA_TRY(run(((1u << bits_) + 255u) / 256u, 0, nwin, wide.size(), bits_));
     }
     for (const Pass &p : passes)
     {
@@ -1071,7 +1135,7 @@ int LdsCircuit::launch(Ctx &ctx, void *state, const std::vector<Pass> &passes)
         ZXA_TRY(ctx.toc(F_FUSED, (p.P.fresh ? 1ull : 2ull) * (uint64_t(1) << bits_) * elem_bytes(prec_)));
         if (tabs)
         {
-            tabs += (size_t(p.P.nwin) << w) * elem_bytes(prec_);
+            tabs += (p.tables() << w) * elem_bytes(prec_);
             factors += tile ? (size_t(p.P.nwin) << p.P.outer) * kFactors : 0;
         }
     }
@@ -1141,7 +1205,7 @@ int LdsCircuit::run(Ctx &ctx, void *state)
             ZXA_TRY(next_pass());
             passes.emplace_back();
             ZXA_TRY(stage(ctx, fresh, passes.back()));
-            tabs += (size_t(passes.back().P.nwin) << passes.back().P.bits) * elem_bytes(prec_);
+            tabs += (passes.back().tables() << passes.back().P.bits) * elem_bytes(prec_);
             fresh = false;
         }
         ZXA_TRY(launch(ctx, state, passes));
