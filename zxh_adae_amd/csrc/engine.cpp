@@ -881,16 +881,20 @@ bool Sim::suits_lds() const
     if (M_ < tile_min_bits(prec_) || (!eager_ && M_ <= 18))
         return true;
     // gates left when each joins the last one on its qubit if nothing has
-    // touched the qubit since
+    // touched the qubit since; windows before a gate; runs of phase gates
     std::vector<uint8_t> touched(N_, 1);
-    size_t left = 0, windows = 0;
-    bool diag = false;
+    size_t left = 0, windows = 0, runs = 0, phases = 0;
+    bool diag = false, cx = false;
     for (const GateRec &g : gates_)
     {
         const bool pairs = g.type == G_H || g.type == G_U3 || (disable_x_ && (g.type == G_X || g.type == G_CX));
+        const bool phase = g.type == G_Z || g.type == G_RZ || g.type == G_P || g.type == G_CP;
         left += pairs && touched[g.q] ? 1u : 0u;
         windows += pairs && diag ? 1u : 0u;
-        diag = pairs ? false : diag || (g.type != G_X && g.type != G_CX);
+        runs += phase && !diag ? 1u : 0u;
+        phases += phase ? 1u : 0u;
+        cx = cx || g.type == G_CX;
+        diag = !pairs && (diag || phase);
         touched[g.q] = !(g.type == G_H || g.type == G_U3);
         if (g.type == G_CP || g.type == G_CX)
             touched[g.cq] = 1;
@@ -898,8 +902,29 @@ bool Sim::suits_lds() const
     // (at the narrowest a layer is one pass of one tile; a QFT, two gates a
     // qubit and a window between any two, takes 142 us against 172 at 20 bits
     // of complex128, where the tile passes form its windows as they go)
-    const bool fans = prec_ != C64 && M_ > 18 && 2 * windows > M_;
-    return 2 * left > (M_ == tile_min_bits(prec_) || fans ? 5 : 3) * M_;
+    const bool c64 = prec_ == C64, narrow = M_ == tile_min_bits(prec_);
+    const bool fans = !c64 && M_ > 18 && 2 * windows > M_;
+    if (2 * left <= (narrow || fans ? 5 : 3) * M_)
+        return false;
+    if (!eager_ || cx)
+        return true;
+    // Whole windows of phase polynomials, which the tile passes take from a
+    // few host coefficients and a table is formed for here, a time that grows
+    // with their gates.  Layers of U3 and n random CP gates and a last layer
+    // of H, against the tile passes (complex128, complex64): two such layers
+    // with 20 gates 0.85, 0.96 of their time at 18 bits and 1.03, 1.12 at 20;
+    // 60 gates 1.00, 1.02 and 1.03, 1.18; 300 gates 1.03, 1.15 and 1.07, 1.19.
+    // One layer, one window: 20 gates 0.97, 1.02 and 1.10, 1.21; 60 gates
+    // 1.06, 1.15 and 1.09, 1.20.  Complex64 of 14 bits, one workgroup's state,
+    // 1.02 to 1.31 throughout; of 13 bits two layers 1.14 and three 0.78.
+    if (narrow)
+        return !c64 || 2 * left > 7 * M_;
+    if (c64 && M_ <= lds_state_bits(prec_))
+        return false;
+    const bool wide = M_ > 18;
+    if (runs == 1)
+        return !c64 && !wide && phases <= 40;
+    return phases <= (c64 ? 48 : wide ? 96 : 384) * runs;
 }
 
 int Sim::execute()
