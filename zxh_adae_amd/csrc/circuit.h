@@ -141,7 +141,7 @@ class LdsCircuit
     }
     std::vector<uint32_t> order_;                 // operations of the pass, by draft
     std::vector<Draft> drafts_;
-    std::vector<uint32_t> vec_, piv_, red_, mix_; // the tile's offsets; elimination
+    std::vector<uint32_t> vec_, piv_, red_;       // the tile's offsets; elimination
     std::vector<uint32_t> pending_, group_;
     std::vector<std::array<uint32_t, 2>> dgates_, ddiags_;
 };

@@ -179,7 +179,7 @@ struct Ctx
     DevBuf scratch_g; // tile-pass per-tile fan factors
     bool timing = false;
     FamilyTiming fam[F_COUNT];
-    // sampler state between prepare and search (tree in scratch_b, tails in scratch_d)
+    // sampler state between launch and search (tree in scratch_b, tails in scratch_d)
     alignas(8) unsigned char sample_levels[64 * 8] = {};
     unsigned sample_m = 0, sample_I = 0;
     bool sample_ready = false;

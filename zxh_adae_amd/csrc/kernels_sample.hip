@@ -671,12 +671,6 @@ int sample_total(Ctx &ctx, double *total)
     return OK;
 }
 
-int sample_prepare(Ctx &ctx, const void *state, int prec, unsigned m, unsigned seg_bits, double *total)
-{
-    ZXA_TRY(sample_launch(ctx, state, prec, m, seg_bits));
-    return sample_total(ctx, total);
-}
-
 // Resolves the thresholds of a sampler launch.  thr, real and pack->out are
 // pinned host memory (the kernel reads and writes them in place); next, when
 // given, forms thresholds [from, to) just before they are searched, so that
@@ -688,7 +682,7 @@ int sample_search(Ctx &ctx, const void *state, int prec, const double *thr, size
         return OK;
     if (!ctx.sample_ready)
     {
-        set_error("sampler: search before prepare");
+        set_error("sampler: search before launch");
         return ESTATE;
     }
     const unsigned m = ctx.sample_m, I = ctx.sample_I;
