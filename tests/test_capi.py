@@ -60,3 +60,16 @@ def test_tuning_knobs_ranges():
         autotune.tune_set(knob, old)
     with pytest.raises(ZXHError):
         autotune.tune_set("no.such.knob", 1)
+
+
+@pytest.mark.skipif(not os.path.exists(_lib.LIB_PATH), reason="native library not built")
+def test_samplers_refuse_null_buffers():
+    """Before a device is looked for: the state is not read."""
+    lib = _lib.load()
+    buf = (ctypes.c_double * 4)()
+    out = (ctypes.c_uint64 * 4)()
+    state = ctypes.cast(buf, ctypes.c_void_p)
+    prec = _lib.ZXH_C128
+    assert lib.zxh_k_sample(state, prec, 1, 18, 5, 4, None) == 1
+    assert lib.zxh_k_sample_thresholds(state, prec, 1, 18, None, 4, out) == 1
+    assert lib.zxh_k_sample_thresholds(state, prec, 1, 18, buf, 4, None) == 1

@@ -622,6 +622,8 @@ int zxh_k_sample(const void *state, int precision, size_t m, size_t seg_bits, ui
         return rc;
     if (shots == 0)
         return ZXH_OK;
+    if (!out_real)
+        return fail(ZXH_EINVAL, "null output");
     WITH_CTX(c);
     return zxa::measure_affine(*c, state, precision, unsigned(m), unsigned(seg_bits), 0, nullptr, nullptr,
                                stream_seed, shots, nullptr, out_real);
@@ -654,6 +656,8 @@ int zxh_k_sample_thresholds(const void *state, int precision, size_t m, size_t s
     int rc = check_kernel_args(state, precision, m);
     if (rc)
         return rc;
+    if (shots && (!thresholds || !out_real))
+        return fail(ZXH_EINVAL, "null pointer");
     WITH_CTX(c);
     return zxa::sample_apply(*c, state, precision, unsigned(m), unsigned(seg_bits), thresholds, shots, out_real);
 }
