@@ -456,7 +456,7 @@ int Ansatz::backward(const double *params, double *grads, double *energy)
     }
     if (nparams_ > 0)
         ZXA_HIP(hipMemcpyAsync(grads, dgrads_, nparams_ * sizeof(double), hipMemcpyDeviceToHost, ctx_.stream));
-    ZXA_HIP(hipStreamSynchronize(ctx_.stream));
+    ZXA_TRY(ctx_.sync());
     return OK;
 }
 

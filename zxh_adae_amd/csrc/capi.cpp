@@ -431,9 +431,7 @@ int zxh_dev_sync(void)
 
 static int finish(zxa::Ctx *c, int rc)
 {
-    if (rc)
-        return rc;
-    return zxa::hip_check(hipStreamSynchronize(c->stream), "stream sync");
+    return rc ? rc : c->sync();
 }
 
 static int check_kernel_args(const void *state, int precision, size_t local_bits)

@@ -131,10 +131,7 @@ void ParamRing::release()
     if (host_)
         (void)hipHostFree(host_);
     dev_ = host_ = hdev_ = nullptr;
-    left_.clear();
-    cur_ = 0;
-    off_ = 0;
-    end_batch();
+    rewind();
 }
 
 // Moves on to the next slot once its last consumers have finished.
@@ -207,6 +204,15 @@ void ParamRing::end_batch()
     batch_ = false;
 }
 
+void ParamRing::rewind()
+{
+    std::fill(used_, used_ + kSlots, false);
+    left_.clear();
+    cur_ = 0;
+    off_ = 0;
+    end_batch();
+}
+
 // Every launch that reads the slots left behind has been made: their events.
 int ParamRing::done(hipStream_t stream)
 {
@@ -234,6 +240,13 @@ int Ctx::init()
     num_cus = prop.multiProcessorCount;
     ZXA_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
     return ring.init();
+}
+
+int Ctx::sync()
+{
+    ZXA_HIP(hipStreamSynchronize(stream));
+    ring.rewind();
+    return OK;
 }
 
 void Ctx::release()

@@ -143,6 +143,10 @@ class ParamRing
     int begin_batch();
     int flush(hipStream_t stream);
     void end_batch();
+    // The stream is idle: from the first slot's start again.  (Blocks at
+    // addresses in recent use: a pass over 12 bits whose table comes to new
+    // ones, 4 MiB of them in turn, took 53 us and not 47.)
+    void rewind();
 
   private:
     int next_slot();
@@ -193,6 +197,8 @@ struct Ctx
         return *reinterpret_cast<T *>(sample_levels);
     }
     int init();
+    // Waits for the stream and hands the parameter ring back.
+    int sync();
     void release();
     ~Ctx()
     {

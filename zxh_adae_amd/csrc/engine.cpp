@@ -1275,7 +1275,7 @@ int Sim::execute()
     ZXA_TRY(flush_pass());
     ZXA_TRY(flush_group());
     ZXA_TRY(settle(size_t(1) << M_));
-    ZXA_HIP(hipStreamSynchronize(ctx_.stream));
+    ZXA_TRY(ctx_.sync());
     executed_ = true;
     return OK;
 }
