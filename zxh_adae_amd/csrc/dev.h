@@ -190,6 +190,7 @@ struct Ctx
     PinBuf sample_total_pin; // the tree root and the search's error flag, written by the kernels
     PinBuf sample_thr_pin;   // thresholds of the kernel-level sampler
     PinBuf sample_out_pin;   // its results
+    PinBuf state_pin;        // get_state output of small states
     template <typename T>
     T &sample_levels_as()
     {

@@ -4,6 +4,7 @@
 #include "dev.h"
 
 #include <algorithm>
+#include <cstring>
 #include <vector>
 
 namespace zxa
@@ -292,6 +293,13 @@ int gather(Ctx &ctx, const void *state, int prec, unsigned n, const uint64_t *id
     return hip_check(e, "gather");
 }
 
+// Widest state whose output the kernel writes to pinned host memory (1 MiB)
+// instead of a device buffer that is then copied: the copy costs 10 us beside
+// its bytes (get_state of 4 qubits 24 us, 14 so, as in a copy of the state and a
+// loop on the host; 12 qubits 50 and 18, the host's loop 58; 16 qubits 101 and
+// 86).  Wider outputs are the same either way and would keep as much pinned.
+constexpr unsigned kPinnedBits = 16;
+
 int virtual_state(Ctx &ctx, const void *state, int prec, unsigned n, unsigned m, const uint64_t *rows,
                   const uint8_t *b, double fx, double fy, double *out)
 {
@@ -343,8 +351,20 @@ int virtual_state(Ctx &ctx, const void *state, int prec, unsigned n, unsigned m,
     }
     const unsigned cbits = std::min(n, 22u); // 64 MiB of output at a time
     const uint64_t chunk = uint64_t(1) << cbits;
-    ZXA_TRY(ctx.scratch_c.ensure(chunk * sizeof(double2)));
-    double2 *dev = static_cast<double2 *>(ctx.scratch_c.ptr);
+    // a small state's output is written to pinned host memory and taken from
+    // there
+    const bool small = n <= kPinnedBits;
+    double2 *dev;
+    if (small)
+    {
+        ZXA_TRY(ctx.state_pin.ensure(chunk * sizeof(double2)));
+        dev = static_cast<double2 *>(ctx.state_pin.ptr);
+    }
+    else
+    {
+        ZXA_TRY(ctx.scratch_c.ensure(chunk * sizeof(double2)));
+        dev = static_cast<double2 *>(ctx.scratch_c.ptr);
+    }
     const unsigned grid = unsigned((chunk + kThreads - 1) / kThreads);
     for (uint64_t first = 0; first < (uint64_t(1) << n); first += chunk)
     {
@@ -359,9 +379,12 @@ int virtual_state(Ctx &ctx, const void *state, int prec, unsigned n, unsigned m,
             hipLaunchKernelGGL(virtual_state_kernel<false>, dim3(grid), dim3(kThreads), 0, ctx.stream, state, m, cols,
                                cbits, w0, fx, fy, dev);
         ZXA_HIP(hipGetLastError());
-        ZXA_HIP(hipMemcpyAsync(out + 2 * first, dev, chunk * sizeof(double2), hipMemcpyDeviceToHost, ctx.stream));
+        if (!small)
+            ZXA_HIP(hipMemcpyAsync(out + 2 * first, dev, chunk * sizeof(double2), hipMemcpyDeviceToHost, ctx.stream));
     }
     ZXA_HIP(hipStreamSynchronize(ctx.stream));
+    if (small)
+        std::memcpy(out, dev, chunk * sizeof(double2));
     return OK;
 }
 
