@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("prec", ["c128", "c64"])
-@pytest.mark.parametrize("n,hs,eager", [(1, 0, False), (3, 1, False), (9, 9, True), (16, 5, False), (17, 5, False), (21, 20, False),
+@pytest.mark.parametrize("n,hs,eager", [(1, 0, False), (3, 1, False), (9, 9, True), (16, 5, False), (18, 5, False), (19, 6, False), (21, 20, False),
                                         (22, 3, False), (23, 4, False), (24, 6, False), (23, 2, True)])
 def test_get_state(gpu_engine, n, hs, eager, prec):
     """hs qubits in superposition, then X, CX, Rz and Z gates (the rows mix,

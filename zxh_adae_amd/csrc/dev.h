@@ -147,6 +147,13 @@ class ParamRing
     // addresses in recent use: a pass over 12 bits whose table comes to new
     // ones, 4 MiB of them in turn, took 53 us and not 47.)
     void rewind();
+    // The slots' host memory (kSlots * kSlotBytes, pinned and coherent) for a
+    // result, right after Ctx::sync(); the device's address of it.
+    void *lend(void **dev) const
+    {
+        *dev = hdev_;
+        return host_;
+    }
 
   private:
     int next_slot();
@@ -190,7 +197,6 @@ struct Ctx
     PinBuf sample_total_pin; // the tree root and the search's error flag, written by the kernels
     PinBuf sample_thr_pin;   // thresholds of the kernel-level sampler
     PinBuf sample_out_pin;   // its results
-    PinBuf state_pin;        // get_state output of small states
     template <typename T>
     T &sample_levels_as()
     {

@@ -293,12 +293,13 @@ int gather(Ctx &ctx, const void *state, int prec, unsigned n, const uint64_t *id
     return hip_check(e, "gather");
 }
 
-// Widest state whose output the kernel writes to pinned host memory (1 MiB)
-// instead of a device buffer that is then copied: the copy costs 10 us beside
-// its bytes (get_state of 4 qubits 24 us, 14 so, as in a copy of the state and a
-// loop on the host; 12 qubits 50 and 18, the host's loop 58; 16 qubits 101 and
-// 86).  Wider outputs are the same either way and would keep as much pinned.
-constexpr unsigned kPinnedBits = 16;
+// Widest state whose output the kernel writes to pinned host memory, that of
+// the parameter ring's slots, instead of a device buffer that is then copied:
+// the copy costs 10 us beside its bytes (get_state of 4 qubits 24 us, 14 so, as
+// in a copy of the state and a loop on the host; 12 qubits 50 and 18, the
+// host's loop 58; 16 qubits 101 and 86, 18 qubits 318 and 280).
+constexpr unsigned kPinnedBits = 18;
+static_assert((sizeof(double2) << kPinnedBits) <= size_t(ParamRing::kSlots) * ParamRing::kSlotBytes, "all slots");
 
 int virtual_state(Ctx &ctx, const void *state, int prec, unsigned n, unsigned m, const uint64_t *rows,
                   const uint8_t *b, double fx, double fy, double *out)
@@ -351,14 +352,15 @@ int virtual_state(Ctx &ctx, const void *state, int prec, unsigned n, unsigned m,
     }
     const unsigned cbits = std::min(n, 22u); // 64 MiB of output at a time
     const uint64_t chunk = uint64_t(1) << cbits;
-    // a small state's output is written to pinned host memory and taken from
-    // there
     const bool small = n <= kPinnedBits;
     double2 *dev;
+    void *host = nullptr;
     if (small)
     {
-        ZXA_TRY(ctx.state_pin.ensure(chunk * sizeof(double2)));
-        dev = static_cast<double2 *>(ctx.state_pin.ptr);
+        ZXA_TRY(ctx.sync());
+        void *p;
+        host = ctx.ring.lend(&p);
+        dev = static_cast<double2 *>(p);
     }
     else
     {
@@ -384,7 +386,7 @@ int virtual_state(Ctx &ctx, const void *state, int prec, unsigned n, unsigned m,
     }
     ZXA_HIP(hipStreamSynchronize(ctx.stream));
     if (small)
-        std::memcpy(out, dev, chunk * sizeof(double2));
+        std::memcpy(out, host, chunk * sizeof(double2));
     return OK;
 }
 
