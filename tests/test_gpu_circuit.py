@@ -1,8 +1,8 @@
 """Circuits executed out of LDS (knobs circuit.bits.<prec>): states of one tile
 (complex128 to 13 address bits, complex64 to 14) and tiles of wider ones,
-against the oracle at the edges of both ranges and of the kernel's step
-chunks, parameter slots, windows and tiles; and the tile passes, which take
-the same circuits when the knob is 0."""
+against the oracle at the edges of both ranges and of a pass's steps, gates,
+windows, window tables and tiles; and the tile passes, which take the same
+circuits when the knob is 0."""
 import numpy as np
 import pytest
 
@@ -50,7 +50,7 @@ def test_soups(gpu_engine, n, mode, prec):
 
 
 @pytest.mark.parametrize("prec", ["c128", "c64"])
-@pytest.mark.parametrize("kind", ["z", "rz", "p", "cp", "cx_cp", "unset"])
+@pytest.mark.parametrize("kind", ["z", "rz", "p", "cp", "cx_cp", "unset", "many"])
 @pytest.mark.parametrize("n", [1, 2, 3, 5])
 def test_no_superposition(gpu_engine, n, kind, prec):
     """Default mode without U3 or H: a state of no address bits, whose phase
@@ -63,7 +63,9 @@ def test_no_superposition(gpu_engine, n, kind, prec):
              "p": [(W.X, 0, b, 0, 0, 0), (W.P, 0, b, 0.3, 0, 0), (W.X, 0, b, 0, 0, 0), (W.P, 0, b, 0.5, 0, 0)],
              "cp": [(W.X, 0, a, 0, 0, 0), (W.X, 0, b, 0, 0, 0), (W.CP, a, b, 0.3, 0, 0)],
              "cx_cp": [(W.X, 0, a, 0, 0, 0), (W.CX, a, b, 0, 0, 0), (W.CP, a, b, 0.3, 0, 0)],
-             "unset": [(W.P, 0, b, 0.3, 0, 0)]}[kind]
+             "unset": [(W.P, 0, b, 0.3, 0, 0)],
+             # (a circuit of up to 24 gates takes a launch of its own for the window)
+             "many": [(W.X, 0, a, 0, 0, 0)] + [(W.X, 0, b, 0, 0, 0), (W.P, 0, b, 0.3, 0, 0)] * 40}[kind]
     s = check(gpu_engine, n, gates, prec, "lazy", (None, 0))
     s.set_seed(5)
     s.measure(7)
@@ -72,7 +74,7 @@ def test_no_superposition(gpu_engine, n, kind, prec):
 
 
 @pytest.mark.parametrize("prec", ["c128", "c64"])
-@pytest.mark.parametrize("n,gates", [(2, [(W.X, 0, 1, 0, 0, 0), (W.P, 0, 1, 0.3, 0, 0)]), (3, W.hadamard_all(3))])
+@pytest.mark.parametrize("n,gates", [(2, [(W.X, 0, 1, 0, 0, 0), (W.P, 0, 1, 0.3, 0, 0)] * 13), (5, W.hadamard_all(5))])
 def test_knob_at_zero_is_never(gpu_engine, n, gates, prec):
     """Also for a state of no address bits."""
     name = f"circuit.bits.{prec}"
@@ -103,9 +105,9 @@ def test_no_gates_and_one_gate(gpu_engine, prec, n):
 @pytest.mark.parametrize("prec", ["c128", "c64"])
 @pytest.mark.parametrize("n,layers", [(4, 120), (7, 700), (13, 60)])
 def test_many_steps(gpu_engine, n, layers, prec):
-    """More steps than one chunk of the kernel's table, than one pass takes
-    (about 500, with the state written and read between the passes), and
-    window tables beyond one pass's share (32 MiB at 13 bits)."""
+    """More steps than one pass takes (about 500, with the state written and
+    read between the passes), and window tables beyond one pass's share (32 MiB
+    at 13 bits)."""
     gates = W.random_layers(n, layers, 40 + n)
     if n == 13:
         # windows that do not merge: one gate between each two
@@ -124,6 +126,21 @@ def test_a_window_larger_than_a_pass_takes(gpu_engine):
     for n in (6, 14):
         window = [g[:3] + (g[3] * 1e-3, 0.0, 0.0) for g in W.diag_batch(n, 9000, 3)]
         check(gpu_engine, n, W.hadamard_all(n) + window + W.hadamard_all(n), "c128", "plain")
+
+
+@pytest.mark.parametrize("prec", ["c128", "c64"])
+@pytest.mark.parametrize("n", [7, 14, 15])
+def test_a_window_of_more_different_gates_than_a_pass_takes(gpu_engine, n, prec):
+    """4000 gates, each under another map (a CX before it), of which a pass
+    takes 2560; a whole state, and tables of every tile.  Angles to 1e-3: see
+    the test above."""
+    r = W.SplitMix64(5 * n)
+    gates = W.hadamard_all(n)
+    for k in range(4000):
+        a, b, c, d = r.below(n), r.below(n - 1), r.below(n), r.below(n - 1)
+        gates.append((W.CX, a, b + (b >= a), 0, 0, 0))
+        gates.append((W.CP, c, d + (d >= c), 1e-3 * r.uniform(), 0, 0))
+    check(gpu_engine, n, gates + W.hadamard_all(n), prec, "lazy", (None, 0))
 
 
 @pytest.mark.parametrize("prec", ["c128", "c64"])
@@ -152,7 +169,7 @@ def test_windows_of_equal_gates(gpu_engine, n, count, mode, prec):
 @pytest.mark.parametrize("n,layers", [(14, 20), (17, 9), (20, 6), (21, 3), (22, 2)])
 def test_layers_over_tiles(gpu_engine, n, layers, prec):
     """Layers with CP ladders: passes that carry parts of several layers, up
-    to eight windows, more steps than one chunk; every state width up to ten
+    to eight windows; every state width up to ten
     address bits outside a tile (the knob at its largest), and more tiles
     than workgroups at a time."""
     top = {"c128": 22, "c64": 23}[prec]

@@ -878,7 +878,8 @@ bool Sim::suits_lds() const
     const size_t widest = size_t(tune_get(prec_ == C64 ? "circuit.bits.c64" : "circuit.bits.c128"));
     if (widest == 0 || M_ > widest)
         return false;
-    if (M_ < tile_min_bits(prec_) || (!eager_ && M_ <= 18))
+    const bool small = M_ < tile_min_bits(prec_) || (!eager_ && M_ <= 18);
+    if (small && gates_.size() > 24)
         return true;
     // gates left when each joins the last one on its qubit if nothing has
     // touched the qubit since; windows before a gate; runs of phase gates
@@ -899,10 +900,15 @@ bool Sim::suits_lds() const
         if (g.type == G_CP || g.type == G_CX)
             touched[g.cq] = 1;
     }
+    const bool c64 = prec_ == C64, narrow = M_ == tile_min_bits(prec_);
+    // A launch or two without tables are quicker (complex128 one H 16 us and 18
+    // here; complex64 16 and 20, two 18.5 and 20, four that grow the state 20
+    // and 21).
+    if (small)
+        return left + runs > (!c64 ? 1u : eager_ || runs ? 2u : 4u);
     // (at the narrowest a layer is one pass of one tile; a QFT, two gates a
     // qubit and a window between any two, takes 142 us against 172 at 20 bits
     // of complex128, where the tile passes form its windows as they go)
-    const bool c64 = prec_ == C64, narrow = M_ == tile_min_bits(prec_);
     const bool fans = !c64 && M_ > 18 && 2 * windows > M_;
     if (2 * left <= (narrow || fans ? 5 : 3) * M_)
         return false;
