@@ -342,7 +342,7 @@ int zxh_ansatz_forward(zxh_ansatz *a, const double *params, double *out);
  * states); re-runs the forward pass unless the last forward used the same
  * params; out (nullable) as in forward.  Uncomputes the device state. */
 int zxh_ansatz_backward(zxh_ansatz *a, const double *params, double *grads, double *out);
-/* device address of the state and its width; tile passes per forward */
+/* device address of the state and its width; sweeps over the state per forward */
 int zxh_ansatz_state(zxh_ansatz *a, void **state, size_t *nbits);
 int zxh_ansatz_passes(zxh_ansatz *a, size_t *tile_passes);
 /* HIP-event timing of the ansatz's own stream (families as zxh_get_timing) */
@@ -369,7 +369,7 @@ int zxh_batch_finalize(zxh_batch *b);
  * (<H>, <psi|psi>); grads (nullable: forward only) concatenated like params */
 int zxh_batch_run(zxh_batch *b, const double *params, double *energies, double *grads);
 int zxh_batch_info(zxh_batch *b, size_t *sets, size_t *total_params, size_t *launches);
-/* one set's width and number of tile passes per forward (after finalize) */
+/* one set's width and number of sweeps per forward (after finalize) */
 int zxh_batch_set_info(zxh_batch *b, size_t set, unsigned *nbits, size_t *passes);
 
 /* tuning knobs (process-wide), set by the autotuner (zxh_adae_amd.autotune):

@@ -43,7 +43,7 @@ constexpr unsigned lds_table_bits(int prec)
 constexpr int kLdsOuter = 10;  // most address bits outside a tile
 constexpr int kLdsWindows = 8; // most windows of a pass over tiles
 
-constexpr int kLdsGates = 3;   // most gates of a step (four, one wave per SIMD, ran 7% slower)
+constexpr int kLdsGates = 3;   // most gates of a step (four, at 256 threads, ran 7% slower)
 
 // A step of the kernel: up to three gates that commute pairwise, or one gate
 // with a control selector, or a diagonal window.  Offsets and selectors are

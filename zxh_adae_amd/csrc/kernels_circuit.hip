@@ -302,19 +302,20 @@ struct CPass
 // (warm_steps) and a window's table entries are loaded before the steps ahead
 // of it run, so no step waits for memory.
 // Bound by its steps.  One of three gates reads and writes the tile once
-// (4096 complex128 amplitudes: 2 x 64 KiB at 128 bytes a cycle), takes 1536
-// FP64 cycles and a barrier, and 1.8 us in all with two workgroups to a
-// compute unit: vector units busy 42% of the time, a third of the wave cycles
-// waiting for LDS or the barrier (the first pass of a 20-qubit U3 + CP-ladder
-// + P circuit, 25 steps and 8 windows: 62 us, of which 12 for a pass without
-// steps and 20 for the multiplications).  What counts is that a launch, its
-// tables and the state's way to memory and back are paid once for many layers:
-// 20 layers of 20 qubits took 41 tile passes at 16 to 21 us, each with a table
-// copy and a factor launch, 980 us in all, and take 11 passes and 620 us here;
-// 10 qubits and 3 layers, whose state is one tile, 30 launches and 205 us, now
-// one and 46 us.
+// (4096 complex128 amplitudes: 2 x 64 KiB at 128 bytes a cycle, 0.43 us), takes
+// 1536 FP64 cycles (0.64 us) and a barrier, and 1.9 us in all: a compute unit
+// holds one workgroup, two waves per SIMD, since two would need four waves and
+// the registers (164; complex64 211) allow three (two), so that little of it
+// overlaps.  20 and 18 bits, 256 and 64 tiles, take the same 1.9 us, 21 bits
+// twice that; complex64, 8192 amplitudes, 2.1; a whole state of 13 bits
+// (complex64 14) 2.3 (3.9).  What counts is that a launch, its tables and the
+// state's way to memory and back are paid once for many layers: 20 layers of 20
+// qubits took 41 tile passes at 16 to 21 us, each with a table copy and a
+// factor launch, 980 us in all, and take 11 passes and 620 us here; 10 qubits
+// and 3 layers, whose state is one tile, 30 launches and 205 us, now one and 46
+// us.
 // kTile: a state of one tile is 2^13 (complex64 2^14) amplitudes, 128 KiB;
-// tiles of a wider one 64 KiB, so that two workgroups share a compute unit.
+// tiles of a wider one 64 KiB.
 constexpr int kLogThreads = 9;
 constexpr int kThreads = 1 << kLogThreads;
 template <bool kC64, bool kTile>
@@ -1111,7 +1112,8 @@ int LdsCircuit::launch(Ctx &ctx, void *state, const std::vector<Pass> &passes)
     {
         const LdsStep *ds = reinterpret_cast<const LdsStep *>(p.steps);
         const LdsDiag *dd = reinterpret_cast<const LdsDiag *>(p.diags);
-        // two workgroups per compute unit (LDS)
+        // (LDS holds two workgroups per compute unit; the registers run them
+        // one after the other)
         const uint32_t nt = std::min(uint32_t(kThreads), std::max(64u, (1u << w) >> 3));
         const uint32_t grid = std::min(p.P.ntiles, 2u * uint32_t(ctx.num_cus > 0 ? ctx.num_cus : 256));
         ZXA_TRY(ctx.tic());

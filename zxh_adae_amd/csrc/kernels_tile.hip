@@ -1586,7 +1586,9 @@ __device__ __forceinline__ void adj_tile(typename UnitT<kC64>::T (&v)[kRegs], ty
 // second round of gates after the window, its rows behind the first round's
 // (28 qubits of complex64: 3.22 ms, two sweeps 2.0 and 2.28; the vector and
 // matrix units are busy for most of it, and for half of a sweep of one round,
-// whose states' way to memory and back is 1.5 ms).
+// whose states' way to memory and back is 1.5 ms).  Two rounds of complex64
+// spill 9 or 10 of 256 VGPRs (40 to 44 bytes of scratch a lane); the other
+// variants none (211 to 256 VGPRs).
 template <bool kC64, bool kL1, bool kL2, bool kDiag, bool kTurn = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void adj_kernel(
     void *__restrict__ psi, void *__restrict__ lam, const TPass P, const TTab *__restrict__ tabp,
