@@ -710,6 +710,23 @@ def test_u3_batch_on_every_qubit_with_the_wide_tile(wide_knobs, prec, n):
     assert passes >= 2
 
 
+@pytest.mark.parametrize("prec,n,first,count", [("c128", 14, 4, 9), ("c128", 18, 1, 14), ("c128", 22, 4, 18),
+                                                ("c64", 15, 5, 10), ("c64", 19, 2, 15), ("c64", 23, 5, 18)])
+def test_u3_batch_with_per_pair_selectors_in_several_passes(wide_knobs, prec, n, first, count):
+    """Single-bit offsets whose selectors see an address bit that no gate of
+    the batch flips (a CX fan-out from a qubit without a gate): more targets
+    than a tile has slots, and selectors that the wide tile does not take."""
+    rng = np.random.default_rng(n + count)
+    psi = rand_state(rng, n)
+    descs = [(pack((1 << q) | (1 if q % 3 else 0), bool(q & 1)), 1 << q, rand_u(rng))
+             for q in range(first, first + count)]
+    want = oracle_u3(psi, n, descs)
+    d = dev(wide_knobs, psi.astype(np.complex64) if prec == "c64" else psi, prec)
+    d.u3_batch(descs)
+    got = d.download().astype(np.complex128)
+    assert np.max(np.abs(got - want)) < (TOL128 if prec == "c128" else TOL64)
+
+
 @pytest.mark.parametrize("prec,n,seed,count,above_run", [
     ("c128", 20, 1, 12, False), ("c128", 22, 2, 17, False), ("c128", 22, 3, 13, True),
     ("c64", 21, 4, 15, False), ("c64", 23, 5, 11, True),

@@ -3859,9 +3859,12 @@ int u3_apply(Ctx &ctx, void *state, int prec, unsigned n, const U3Gate *gates, s
     }
     // single-bit batches: the first pass as planned, the remaining targets in
     // wide passes of nine when that takes no more passes (their runs are
-    // longer)
+    // longer), which take no selector besides the target's bit
     std::vector<bool> wide13(best.size(), false);
-    if (wide.empty() && best.size() >= 2)
+    const bool plain = std::all_of(single.begin(), single.end(), [](const U3Gate *g) {
+        return (g->packed_sel & ((uint64_t(1) << 63) - 1)) == g->delta;
+    });
+    if (wide.empty() && plain && best.size() >= 2)
     {
         // the first pass as a 4096-unit tile pass, the others wide
         // (tile_layer_plan)
