@@ -922,10 +922,11 @@ bool Sim::suits_lds() const
     // 60 gates 1.00, 1.02 and 1.03, 1.18; 300 gates 1.03, 1.15 and 1.07, 1.19.
     // One layer, one window: 20 gates 0.97, 1.02 and 1.10, 1.21; 60 gates
     // 1.06, 1.15 and 1.09, 1.20.  Complex64 of 14 bits, one workgroup's state,
-    // 1.02 to 1.31 throughout; of 13 bits two layers 1.14 and three 0.78.
+    // 1.02 to 1.31 for up to four layers, 0.97 for eight with a ladder each; of
+    // 13 bits two layers and one of H 1.14, three 0.81 to 0.98.
     if (narrow)
-        return !c64 || 2 * left > 7 * M_;
-    if (c64 && M_ <= lds_state_bits(prec_))
+        return !c64 || runs >= 3 || 2 * left > 7 * M_;
+    if (c64 && M_ <= lds_state_bits(prec_) && left < 8 * M_)
         return false;
     const bool wide = M_ > 18;
     if (runs == 1)

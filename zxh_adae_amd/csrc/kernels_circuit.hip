@@ -318,7 +318,8 @@ struct CPass
 // tiles of a wider one 64 KiB.
 constexpr int kLogThreads = 9;
 constexpr int kThreads = 1 << kLogThreads;
-template <bool kC64, bool kTile>
+// kFull: some window has a table of every tile (P.wfull).
+template <bool kC64, bool kTile, bool kFull = false>
 __global__ __launch_bounds__(kThreads) void circuit_kernel(typename CGeo<kC64>::T *__restrict__ state, const CPass P,
                                                            const LdsStep *__restrict__ steps,
                                                            const LdsDiag *__restrict__ diags,
@@ -404,7 +405,7 @@ __global__ __launch_bounds__(kThreads) void circuit_kernel(typename CGeo<kC64>::
             {
                 const uint32_t wi = min(win, P.nwin - 1);
                 uint64_t table = wi;
-                if constexpr (kTile)
+                if constexpr (kFull)
                     table += uint64_t(__builtin_popcount(P.wfull & ((1u << wi) - 1))) * (P.ntiles - 1) +
                              ((P.wfull >> wi) & 1u ? tile : 0u);
                 src = tabs + (table << P.bits);
@@ -1117,8 +1118,10 @@ int LdsCircuit::launch(Ctx &ctx, void *state, const std::vector<Pass> &passes)
         const uint32_t nt = std::min(uint32_t(kThreads), std::max(64u, (1u << w) >> 3));
         const uint32_t grid = std::min(p.P.ntiles, 2u * uint32_t(ctx.num_cus > 0 ? ctx.num_cus : 256));
         ZXA_TRY(ctx.tic());
+        const bool full = p.P.wfull != 0;
         if (c64 && tile)
-            hipLaunchKernelGGL((circuit_kernel<true, true>), dim3(grid), dim3(nt), 0, ctx.stream,
+            hipLaunchKernelGGL((full ? circuit_kernel<true, true, true> : circuit_kernel<true, true, false>),
+                               dim3(grid), dim3(nt), 0, ctx.stream,
                                static_cast<float2 *>(state), p.P, ds, dd, reinterpret_cast<const float2 *>(tabs),
                                factors);
         else if (c64)
@@ -1126,7 +1129,8 @@ int LdsCircuit::launch(Ctx &ctx, void *state, const std::vector<Pass> &passes)
                                static_cast<float2 *>(state), p.P, ds, dd, reinterpret_cast<const float2 *>(tabs),
                                factors);
         else if (tile)
-            hipLaunchKernelGGL((circuit_kernel<false, true>), dim3(grid), dim3(nt), 0, ctx.stream,
+            hipLaunchKernelGGL((full ? circuit_kernel<false, true, true> : circuit_kernel<false, true, false>),
+                               dim3(grid), dim3(nt), 0, ctx.stream,
                                static_cast<double2 *>(state), p.P, ds, dd,
                                reinterpret_cast<const double2 *>(tabs), factors);
         else
